@@ -76,6 +76,27 @@ __device__ __forceinline__ float col_sum4(float x) {
   return a + b;
 }
 
+// max / sum over the wave's 64 lanes, in every lane: rotations within rows of
+// 16 lanes by DPP, then across the rows (no LDS).  Every lane must be active.
+template <int N>
+__device__ __forceinline__ float row_ror(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + N, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float wave_max(float x) {
+  x = fmaxf(x, row_ror<8>(x));
+  x = fmaxf(x, row_ror<4>(x));
+  x = fmaxf(x, row_ror<2>(x));
+  x = fmaxf(x, row_ror<1>(x));
+  return col_max4(x);
+}
+__device__ __forceinline__ float wave_sum(float x) {
+  x += row_ror<8>(x);
+  x += row_ror<4>(x);
+  x += row_ror<2>(x);
+  x += row_ror<1>(x);
+  return col_sum4(x);
+}
+
 // RoPE (transformers' apply_rotary_pos_emb: x*cos + rotate_half(x)*sin) of 8
 // dims i (lo) and their partners i + D/2 (hi): lo' = lo*c_lo - hi*s_lo,
 // hi' = hi*c_hi + lo*s_hi.  A product of two fp16 values is exact in fp32, so

@@ -213,9 +213,10 @@ struct PartRows {
 constexpr int kPlanDescWords = 8;
 constexpr int kPlanWaves = 4;
 
-template <int D, int NTHREADS>
+template <int D, int NTHREADS, bool kMany>
 __device__ __forceinline__ void merge_splits(const DecodeParams& p, const PartRows& prow, int b,
-                                             int g, int n_states, int tid);
+                                             int g, int n_splits, int n_states, int tid,
+                                             f32x4* sm);
 
 // Profiling builds only (-DCIE_DECODE_TRACE): phase boundaries
 // (s_memrealtime) are stamped into LDS — LDS writes do not count in vmcnt, so
@@ -268,7 +269,7 @@ __device__ uint64_t* g_decode_trace;
 // preloaded into SGPRs (the build's kernel-argument preload count), so that
 // load goes out without waiting for the kernel-argument load (-0.1 to
 // -0.4 us per call).
-template <int D, int WAVES, bool kAppend, bool kRope, bool kPlanned>
+template <int D, int WAVES, bool kAppend, bool kRope, bool kPlanned, bool kMany>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1)))
 void decode_kernel(const int64_t* __restrict__ a_slot_ids, const int32_t* __restrict__ a_plan,
                    int32_t a_n_wg, DecodeParams p) {
@@ -582,6 +583,15 @@ void decode_kernel(const int64_t* __restrict__ a_slot_ids, const int32_t* __rest
 
   DECODE_TRACE(2, __builtin_amdgcn_s_memrealtime());
   DECODE_TRACE_LANE0(16 + wave, __builtin_amdgcn_s_memrealtime());
+  // Splits that hold a tile: with at most one tile a wave the deal gives split
+  // s the tiles [s * WAVES, (s + 1) * WAVES), so the splits from this one on
+  // are empty.  They arrive (the counter counts all S) but write no partial,
+  // and the merge reads only the others'.  (A plan deals no empty splits; a
+  // launch of few splits merges them all.)
+  const int S_used = kPlanned || !kMany
+                         ? S
+                         : min(S, max(1, (uniform(opaque(n_tiles)) + WAVES - 1) / WAVES));
+  if (split < S_used) {  // uniform
   // Fold the waves of this workgroup.  Lane (r16, grp) holds dims
   // NT*(4*grp + r) + nt of column r16: for each r, NT consecutive dims, written
   // as NT/4 16-byte vectors.  One thread then folds 4 dims of one head.
@@ -633,6 +643,7 @@ void decode_kernel(const int64_t* __restrict__ a_slot_ids, const int32_t* __rest
       }
     }
   }
+  }
   DECODE_TRACE(9, __builtin_amdgcn_s_memrealtime());
   if (S == 1) {
     if constexpr (!kRope) store_odd();
@@ -649,27 +660,27 @@ void decode_kernel(const int64_t* __restrict__ a_slot_ids, const int32_t* __rest
     DECODE_TRACE_DUMP();
     return;
   }
-  merge_splits<D, WAVES * kWave>(p, prow, b, g, S, threadIdx.x);
+  merge_splits<D, WAVES * kWave, kMany>(p, prow, b, g, S, S_used, threadIdx.x, &sm_acc[0][0][0]);
   if (threadIdx.x == 0) counter_reset(arrival);
   DECODE_TRACE(4, __builtin_amdgcn_s_memrealtime());
   DECODE_TRACE_DUMP();
 }
 
-// Combine the S partial states of every head of (b, g) into o.  A thread
-// owns 4 dims of one head and takes the splits in groups of kMergeGroup: the m, l
-// and acc loads of a group are all issued before any is used (one memory round
-// trip per group), and a running log-sum-exp carries across groups.  For
-// S <= kMergeGroup the arithmetic is the plain max-then-sum of
-// kernels/decode_attention.py:243-264.
+// Combine the first n_states of the n_splits partial states of every head of
+// (b, g) into o.  A thread owns 4 dims of one head and takes the states in
+// groups of kMergeGroup: the m, l and acc loads of a group are all issued before
+// any is used (one memory round trip per group), and a running log-sum-exp
+// carries across groups.  For up to kMergeGroup states the arithmetic is the
+// plain max-then-sum of kernels/decode_attention.py:243-264.
 constexpr int kMergeGroup = 8;
 
 template <int D, int NTHREADS>
-__device__ __forceinline__ void merge_splits(const DecodeParams& p, const PartRows& prow, int b,
-                                             int g, int n_states, int tid) {
+__device__ __forceinline__ void merge_few(const DecodeParams& p, const PartRows& prow, int b, int g,
+                                          int n_splits, int n_states, int tid) {
   constexpr int D4 = D / 4;
   const int S = n_states;
   const __amdgpu_buffer_rsrc_t racc =
-      coherent_rsrc(p.part_acc + prow.base * D, (uint32_t)(p.G * S * D * sizeof(float)));
+      coherent_rsrc(p.part_acc + prow.base * D, (uint32_t)(p.G * n_splits * D * sizeof(float)));
   for (int it = tid; it < p.G * D4; it += NTHREADS) {
     const int h = it / D4;
     const int d4 = it - h * D4;
@@ -714,6 +725,106 @@ __device__ __forceinline__ void merge_splits(const DecodeParams& p, const PartRo
   }
 }
 
+// The same for any number of states.  One workgroup merges, so it is bound by
+// memory round trips (the partials come from other XCDs) and by how many loads
+// it keeps in flight.  A thread owns 4 dims of one head and every
+// R-th split, R = threads / (G * D / 4); its first kMergeLoads acc loads go out
+// together with the m and l loads.  Those take one split a lane (kMaxSplits =
+// the wave): a wave reduces a head's max and sum across lanes, and the splits'
+// weights 2^(m - M) / l go to LDS, so no thread repeats them.
+// sm: 16 * kMaxSplits floats of weights, then NTHREADS f32x4 of partial sums.
+constexpr int kMergeLoads = 16;
+
+template <int D, int NTHREADS>
+__device__ __forceinline__ void merge_many(const DecodeParams& p, const PartRows& prow, int b, int g,
+                                           int n_splits, int n_states, int tid, f32x4* sm) {
+  static_assert(kMaxSplits == kWave, "a split per lane");
+  constexpr int D4 = D / 4;
+  constexpr int NW = NTHREADS / kWave;
+  constexpr int kHeads = (16 + NW - 1) / NW;  // heads a wave weighs at most
+  const int S = n_states;
+  float* const sm_w = reinterpret_cast<float*>(sm);  // [head][split]
+  f32x4* const sm_sum = sm + 16 * kMaxSplits / 4;    // [thread]
+  const int lane = tid & (kWave - 1), wave = tid / kWave;
+  const __amdgpu_buffer_rsrc_t racc =
+      coherent_rsrc(p.part_acc + prow.base * D, (uint32_t)(p.G * n_splits * D * sizeof(float)));
+  float ms[kHeads], ls[kHeads];
+#pragma unroll
+  for (int i = 0; i < kHeads; ++i) {
+    const int h = wave + i * NW;
+    ms[i] = kNegInf;
+    ls[i] = 0.f;
+    if (h < p.G && lane < S) {
+      const int row = prow.rel(h, lane);
+      ms[i] = partial_load(&p.part_m[prow.base + row]);
+      ls[i] = partial_load(&p.part_l[prow.base + row]);
+    }
+  }
+  const int n_units = p.G * D4;
+  const int R = max(1, NTHREADS / n_units);  // threads per unit
+  for (int u0 = 0; u0 < n_units; u0 += NTHREADS) {
+    const int r = tid / n_units;
+    const int unit = u0 + (R > 1 ? tid - r * n_units : tid);
+    const bool live = unit < n_units && r < R;
+    const int h = live ? unit / D4 : 0;
+    const int d4 = unit - h * D4;
+    f32x4 num = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = r; s0 < S || s0 == r; s0 += R * kMergeLoads) {
+      f32x4 as[kMergeLoads];
+#pragma unroll
+      for (int u = 0; u < kMergeLoads; ++u) {
+        // past the last split: beyond the descriptor, which reads zeros
+        const int s = s0 + u * R;
+        const uint32_t off = live && s < S ? (uint32_t)((prow.rel(h, s) * D + 4 * d4) * sizeof(float))
+                                           : 0x7ffffff0u;
+        as[u] = agent_load4(racc, off);
+      }
+      if (u0 == 0 && s0 == r) {
+#pragma unroll
+        for (int i = 0; i < kHeads; ++i) {
+          const int hh = wave + i * NW;
+          if (hh < p.G) {  // uniform in the wave
+            const float M = wave_max(ms[i]);
+            const float a = ms[i] == kNegInf ? 0.f : fast_exp2(ms[i] - M);
+            const float den = wave_sum(a * ls[i]);
+            sm_w[hh * kMaxSplits + lane] = den > 0.f ? a / den : 0.f;  // no key at all: o = 0
+          }
+        }
+        __syncthreads();
+      }
+#pragma unroll
+      for (int u = 0; u < kMergeLoads; ++u) {
+        const int s = s0 + u * R;
+        num += (s < S ? sm_w[h * kMaxSplits + s] : 0.f) * as[u];
+      }
+    }
+    if (R > 1) {  // uniform; one pass over the units then
+      sm_sum[tid] = num;
+      __syncthreads();
+      if (r > 0 || !live) continue;
+      for (int i = 1; i < R; ++i) num += sm_sum[tid + i * n_units];
+    }
+    if (!live) continue;
+    const f16x4 o4 = {(f16)num[0], (f16)num[1], (f16)num[2], (f16)num[3]};
+    *reinterpret_cast<f16x4*>(p.o + ((int64_t)b * p.H_q + g * p.G + h) * D + 4 * d4) = o4;
+  }
+}
+
+// kMany kernels take the second from kMergeFew states up (64 splits of 2 x
+// 98,000 keys: 26.3 us a call when eight rounds of 8 followed each other, 23.4;
+// 16 splits of 1 x 1,000 keys: 6.8 through the first, 7.3).
+constexpr int kMergeFew = 16;
+
+template <int D, int NTHREADS, bool kMany>
+__device__ __forceinline__ void merge_splits(const DecodeParams& p, const PartRows& prow, int b,
+                                             int g, int n_splits, int n_states, int tid,
+                                             f32x4* sm) {
+  if (!kMany || n_states <= kMergeFew)
+    merge_few<D, NTHREADS>(p, prow, b, g, n_splits, n_states, tid);
+  else
+    merge_many<D, NTHREADS>(p, prow, b, g, n_splits, n_states, tid, sm);
+}
+
 // ---------------------------------------------------------------------------
 // A decode step's plan.  The slot ids, lengths and block-table rows a decode
 // reads are the same for every layer of a step (the lengths advance after
@@ -724,8 +835,8 @@ __device__ __forceinline__ void merge_splits(const DecodeParams& p, const PartRo
 // descriptor and its waves' page ids) before its first K/V loads, where an
 // unplanned one needs two (slot id, then page ids and length).
 //
-// Splits are balanced by length: tau, the smallest tile count per split for
-// which sum_b max(1, ceil(tiles_b / tau)) splits (at most kMaxSplits each)
+// Splits are balanced by length: tau, the smallest tile count per split (at
+// least a tile per wave: more splits would be empty) for which sum_b max(1, ceil(tiles_b / tau)) splits (at most kMaxSplits each)
 // fit the grid's n_wg / H_kv workgroups per kv head, gives sequence b
 // ceil(tiles_b / tau) splits, so the longest sequences no longer set the call
 // when lengths differ.  Equal lengths get equal splits (the unplanned deal).
@@ -844,7 +955,7 @@ __device__ __forceinline__ void plan_wave(const PlanParams& p) {
     for (int off = 1; off < kWave; off <<= 1) c += __shfl_xor(c, off, kWave);
     return c <= n_ph;
   };
-  int lo = max(1, (total + n_ph - 1) / n_ph);
+  int lo = max(kPlanWaves, (total + n_ph - 1) / n_ph);
   hi = max(hi, lo);
   if (!fits(lo)) {  // binary search in (lo, hi]; hi always fits (one split each)
     while (lo + 1 < hi) {
@@ -918,7 +1029,8 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams p)
   // 2. the smallest tiles-per-split tau whose splits fit n_wg / H_kv per kv head
   const int n_ph = p.n_wg / p.H_kv;
   auto splits_of = [](int nt, int tau) { return plan_splits(nt, tau); };
-  int lo = 1;
+  int lo = kPlanWaves;
+  hi = max(hi, lo);
   while (lo < hi) {  // uniform: every thread holds the same bounds
     const int mid = (lo + hi) >> 1;
     int c = 0;
@@ -1010,26 +1122,37 @@ static int device_cus() {
   return cus[dev];
 }
 
-template <int D, int W, bool kAppend, bool kRope>
-static int launch_decode_waves(const DecodeParams& p, hipStream_t stream) {
-  dim3 grid(p.n_splits, p.H_kv, p.B);
-  hipLaunchKernelGGL((decode_kernel<D, W, kAppend, kRope, false>), grid, dim3(W * kWave), 0, stream,
-                     p.slot_ids, p.plan, p.n_wg, p);
+template <int D, int W, bool kAppend, bool kRope, bool kPlanned, bool kMany>
+static int launch_decode_kernel(const DecodeParams& p, hipStream_t stream) {
+  // planned: one workgroup per plan entry
+  const dim3 grid = kPlanned ? dim3(p.n_wg) : dim3(p.n_splits, p.H_kv, p.B);
+  hipLaunchKernelGGL((decode_kernel<D, W, kAppend, kRope, kPlanned, kMany>), grid, dim3(W * kWave), 0,
+                     stream, p.slot_ids, p.plan, p.n_wg, p);
   return (int)hipGetLastError();
+}
+
+// kMany (merge_many compiled in) only for launches that deal more than
+// kMergeFew splits a (sequence, kv head), on average for a planned one: its
+// code in the others' kernels costs them 1-2 % (32 x 4,096 keys in 4 splits:
+// 17.2 us a call against 16.9).  A planned launch of fewer whose longest
+// sequence gets more merges them in rounds of kMergeGroup.
+template <int D, int W, bool kAppend, bool kRope, bool kPlanned>
+static int launch_decode_waves(const DecodeParams& p, hipStream_t stream) {
+  const bool many = kPlanned ? (int64_t)p.n_wg > (int64_t)kMergeFew * p.B * p.H_kv : p.n_splits > kMergeFew;
+  return many ? launch_decode_kernel<D, W, kAppend, kRope, kPlanned, true>(p, stream)
+              : launch_decode_kernel<D, W, kAppend, kRope, kPlanned, false>(p, stream);
 }
 
 template <int D, bool kAppend, bool kRope, bool kPlanned>
 static int launch_decode(const DecodeParams& p, hipStream_t stream) {
-  if constexpr (kPlanned) {  // one workgroup per plan entry, kPlanWaves waves each
-    hipLaunchKernelGGL((decode_kernel<D, kPlanWaves, kAppend, kRope, true>), dim3(p.n_wg),
-                       dim3(kPlanWaves * kWave), 0, stream, p.slot_ids, p.plan, p.n_wg, p);
-    return (int)hipGetLastError();
+  if constexpr (kPlanned) {
+    return launch_decode_waves<D, kPlanWaves, kAppend, kRope, true>(p, stream);
   } else {
     constexpr int W = decode_waves<D>();
     constexpr int Wh = W > 4 ? W / 2 : W;
     const int64_t n_wg = (int64_t)p.n_splits * p.H_kv * p.B;
-    return (Wh != W && n_wg > device_cus()) ? launch_decode_waves<D, Wh, kAppend, kRope>(p, stream)
-                                            : launch_decode_waves<D, W, kAppend, kRope>(p, stream);
+    return (Wh != W && n_wg > device_cus()) ? launch_decode_waves<D, Wh, kAppend, kRope, false>(p, stream)
+                                            : launch_decode_waves<D, W, kAppend, kRope, false>(p, stream);
   }
 }
 

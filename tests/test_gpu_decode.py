@@ -255,3 +255,20 @@ def test_decode_counter_preloaded_negative_is_flagged_then_reset(native_lib):
         assert int(err.item()) == 0
         assert torch.count_nonzero(ctr) == 0
         assert_attn_close(o[0].float().cpu(), want, what="call after the reset")
+
+
+@pytest.mark.parametrize("h_q,h_kv,d", [(14, 2, 64), (16, 1, 64), (2, 2, 64), (8, 1, 128), (16, 1, 128)])
+@pytest.mark.parametrize("splits", [16, 17, 33, 64])
+def test_decode_merge_of_many_splits(native_lib, h_q, h_kv, d, splits):
+    """More than 16 splits merge through the kernel that weighs a split a lane:
+    lengths that leave splits empty (1 to 65 tiles of 4 a workgroup), that give
+    every wave one tile and several, and each number of threads a unit
+    (2 to 16 heads, D = 64 and 128: 16 to 1, and two passes of the units)."""
+    case = inputs.make_case([0, 1, 63, 64, 1000, 1040, 4200], seed=61, h_q=h_q, h_kv=h_kv, d=d)
+    note(f"many splits {splits} {h_q}/{h_kv} D={d}")
+    err = err_word()
+    kp, vp, o = gpu_decode_fused_step(case, n_splits=splits, err=err)
+    assert int(err.item()) == 0
+    ko, vo = case.appended_pools()
+    assert torch.equal(bits(kp), bits(ko)) and torch.equal(bits(vp), bits(vo))
+    assert_attn_close(o, oracle_decode(case), what="many splits")
