@@ -185,7 +185,8 @@ int cie_paged_decode_append(void* o, const void* q, void* k_pool, void* v_pool,
  * as the layers' calls, and n_workgroups must be the same for all of them.
  * n_workgroups = cie_paged_decode_plan_workgroups(B, H_kv, n_splits):
  * B * H_kv * n_splits, or with n_splits = 0 the library's default (about
- * one workgroup per CU, at least one per (sequence, kv head)); it must lie
+ * one workgroup per CU, or the whole number per CU that gives every (sequence,
+ * kv head) at least one); it must lie
  * in [B * H_kv, B * H_kv * cie_paged_decode_max_splits()] and be a multiple
  * of H_kv.  Equal lengths give every (sequence, kv head) n_workgroups /
  * (B * H_kv) splits; unequal ones give longer sequences more.  partials:
