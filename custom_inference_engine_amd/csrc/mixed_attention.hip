@@ -8,6 +8,10 @@
 // (the causal rule kv_len + row >= key of prefill_attention.py:145-146).
 // Rows outside every sequence are left untouched.
 //
+// Launches with enough prefill rows to fill the chip run wide items
+// (wide_tiles.h, wide_rule); what follows is the others', and the decode rows
+// of both.
+//
 // Work.  A sequence's rows are cut into 16-row query tiles (the reference's
 // BLOCK_M; grid (cdiv(max_seqlen, 16), H_kv, B), attn/core.py:90).  A tile's
 // work is laid out as (row, head) columns, G heads per row, packed 16 to an
@@ -33,7 +37,7 @@
 // mixed_plan_kernel, instead.  The reference instead walks a tile's whole
 // prefix with one program and pads every L = 1 sequence to a 16-row tile
 // (prefill_attention.py:49-50, 93).
-#include "attn_engine.h"
+#include "wide_tiles.h"
 
 namespace cie {
 
@@ -101,6 +105,7 @@ namespace cie {
 
 constexpr int kWavePairs = CIE_MIXED_WAVE_PAIRS;
 constexpr int kMaxChunks = 16;    // workgroups per (tile, column group) at most
+constexpr int kWideWeight = 3;    // cost of a wide item's key tile, in a narrow item's
 constexpr int kMaxColGroups = 8;  // column groups per tile at most (<= 8 column tiles)
 // Partial rows a launch uses at most, whatever the buffer: with each
 // sequence's rows clamped to the budget + 1, the plan's prefix over kMaxSeqs
@@ -163,6 +168,8 @@ struct MixedParams {
   int32_t bt_width, n_slots, B, H_q, H_kv, G, page_size, n_qtiles;
   uint32_t g_magic, tpp_magic;  // div_magic(G), div_magic(page_size / 16)
   uint32_t pool_bytes;          // bytes of each pool if under 4 GiB, else 0
+  int32_t wide_m;  // 16-row blocks of a wide query tile (wide_rule); 0: the launch has none
+  int32_t wide_wg;  // workgroups of a wide launch
   float scale_log2;
   int32_t* err;
   // planned launches: the step's plan (cie_mixed_plan) and its capacity in
@@ -180,10 +187,21 @@ struct SeqInfo {
   // first partial row of the sequence's split tiles, or -1: its tiles are
   // not split (the batch's partial rows would exceed the caller's buffer)
   int pbase;
+  int m;  // wide query tiles: their 16-row blocks (seq_blocks); 0: tiles of 16 rows
+  int q;  // wide query tiles of more key tiles than this are two chunks (wide_share)
 };
 
+// In a wide launch every sequence of more than one column tile is cut into
+// wide tiles.
+__device__ __forceinline__ int seq_rows(const MixedParams& p, int L) {
+  return min((int64_t)L, (int64_t)p.n_qtiles * 16);  // rows computed (the max_seqlen cap)
+}
+__device__ __forceinline__ int seq_blocks(const MixedParams& p, int L) {
+  return p.wide_m > 0 && seq_rows(p, L) * p.G > 16 ? p.wide_m : 0;
+}
+
 __device__ __forceinline__ SeqInfo seq_info(const MixedParams& p, int b) {
-  SeqInfo s{0, 0, 0, 0, 0};
+  SeqInfo s{0, 0, 0, 0, 0, 0, 0};
   const int64_t t0 = p.cu_seqlens[b];
   const int64_t t1 = p.cu_seqlens[b + 1];
   const int64_t slot = p.slot_ids[b];
@@ -201,6 +219,7 @@ __device__ __forceinline__ SeqInfo seq_info(const MixedParams& p, int b) {
   s.slot = slot;
   s.L = (int)(t1 - t0);
   s.c = (int)c;
+  s.m = seq_blocks(p, s.L);
   return s;
 }
 
@@ -240,21 +259,24 @@ __device__ __forceinline__ int n_col_groups(int n, int cg) {
 // walks its sequence's tiles, and a run-time division per tile cost ~2 us on
 // the last tiles of a 2,304-key sequence).
 template <int CG, int W>
-__device__ __forceinline__ TilePlan tile_plan(int qt, const SeqInfo& s, int G) {
+__device__ __forceinline__ TilePlan tile_plan(const MixedParams& p, int qt, const SeqInfo& s) {
   TilePlan t;
-  t.row0 = qt * 16;
-  t.rows = min(16, s.L - t.row0);
-  t.n_combos = t.rows * G;
+  const bool wide = s.m > 0;
+  const int block = wide ? 16 * s.m : 16;
+  t.row0 = qt * block;
+  t.rows = min(block, (wide ? seq_rows(p, s.L) : s.L) - t.row0);
+  t.n_combos = t.rows * p.G;
   t.n_ctiles = (t.n_combos + 15) >> 4;
-  t.cg = seq_cg<CG>(s);
-  t.n_groups = n_col_groups<CG>(t.n_ctiles, t.cg);
+  t.cg = wide ? kWideColTiles : seq_cg<CG>(s);
+  t.n_groups = wide ? 1 : n_col_groups<CG>(t.n_ctiles, t.cg);
   t.key_end = s.c + t.row0 + t.rows;
   t.n_ktiles = (t.key_end + 15) >> 4;
   t.n_pairs = (t.n_ktiles + 1) >> 1;
   constexpr int kPerNarrow = W * CIE_MIXED_NARROW_PAIRS;
   constexpr int kPerWide = W * kWavePairs;
-  const int chunks = t.n_ctiles == 1 ? (t.n_pairs + kPerNarrow - 1) / kPerNarrow
-                                     : (t.n_pairs + kPerWide - 1) / kPerWide;
+  const int chunks = wide ? (t.n_ktiles > s.q ? 2 : 1)
+                     : t.n_ctiles == 1 ? (t.n_pairs + kPerNarrow - 1) / kPerNarrow
+                                       : (t.n_pairs + kPerWide - 1) / kPerWide;
   t.n_chunks = s.pbase < 0 ? 1 : max(1, min(kMaxChunks, chunks));
   t.pblk = 0;
   return t;
@@ -538,6 +560,55 @@ __device__ __forceinline__ void run_group(const MixedParams& p, const SeqInfo& s
   }
 }
 
+// One wide item's wave: key tiles [kt0, kt1) against column tiles
+// [ct0, ct0 + NCT) of the tile (those past its last column hold zeros), o or
+// the chunk's partial state written from the wave's registers.
+template <int D, int NCT>
+__device__ __forceinline__ void run_wide(const MixedParams& p, const SeqInfo& s, const TilePlan& tp,
+                                         int g, int ct0, int chunk, int kt0, int kt1,
+                                         const PagedSrc& src, int r16, int grp, f16* sm) {
+  constexpr int NT = Geo<D>::NT;
+  SoftmaxAcc<D, NCT> st;
+  st.init();
+  f16x8 q[NCT][Geo<D>::KS];
+  int lim[NCT];
+#pragma unroll
+  for (int c = 0; c < NCT; ++c) load_combo_q<D>(p, s, tp, g, ct0 + c, r16, grp, q[c], lim[c]);
+  const bool live = ct0 < tp.n_ctiles;
+  stream_wide<D, NCT>(st, q, lim, kt0, kt1, tp.key_end, src, p.scale_log2, sm);
+  if (!live) return;
+  const int lane = opaque((int)threadIdx.x) & (kWave - 1);
+  r16 = lane & 15;
+  grp = lane >> 4;
+  const int64_t tile_row0 = (s.t0 + tp.row0) * p.H_q;
+  const PartRegion pr = part_region<D>(p, tp);  // (used only if tp.n_chunks > 1)
+#pragma unroll
+  for (int c = 0; c < NCT; ++c) {
+    const float l = st.l(c);  // (every lane takes part)
+    const int cc = (ct0 + c) * 16 + r16;
+    if (cc >= tp.n_combos) continue;
+    const int off = column_off(p, g, cc);
+    if (tp.n_chunks == 1) {
+      const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const f32x4 a = st.acc[c][nt] * inv;
+        *reinterpret_cast<f16x4*>(p.o + (tile_row0 + off) * D + 16 * nt + 4 * grp) =
+            f16x4{(f16)a[0], (f16)a[1], (f16)a[2], (f16)a[3]};
+      }
+    } else {
+      const int prow = off * tp.n_chunks + chunk;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+        agent_store4(pr.acc, (uint32_t)((prow * D + 16 * nt + 4 * grp) * sizeof(float)), st.acc[c][nt]);
+      if (grp == 0) {
+        agent_store(pr.m + prow, st.m[c]);
+        agent_store(pr.l + prow, l);
+      }
+    }
+  }
+}
+
 // Last chunk of a (tile, column group): combine the n_chunks partials of the
 // group's columns into o.  A unit is 4 consecutive dims of one column
 // (consecutive threads: consecutive dims, so every load is a whole-line
@@ -545,12 +616,12 @@ __device__ __forceinline__ void run_group(const MixedParams& p, const SeqInfo& s
 // chunks, issues the loads of all of them before combining any, so a merge
 // of up to four chunks is one memory round trip; chunks are combined with a
 // running log-sum-exp.
-template <int D>
+template <int D, int CT>
 __device__ __forceinline__ void merge_group(const MixedParams& p, const SeqInfo& s,
                                             const TilePlan& tp, int g, int ct0, int n_cols) {
   constexpr int kGroup = 4;
   constexpr int NTH = mixed_waves<D>() * kWave;
-  constexpr int kUnits = (16 * col_group<D>() * (D / 4) + NTH - 1) / NTH;
+  constexpr int kUnits = (16 * CT * (D / 4) + NTH - 1) / NTH;
   const int K = tp.n_chunks;
   const int n_units = n_cols * (D / 4);
   const int64_t tile_row0 = (s.t0 + tp.row0) * p.H_q;
@@ -645,25 +716,40 @@ constexpr size_t kLdsPerWorkgroup = 160 * 1024;
 // count that are counted and searched without walking the tiles.  A
 // sequence's items are walked heaviest first: its partial last tile (if
 // any), then its full tiles from the top down.
+// Wide tiles (16 * m rows) follow the same rules with m key tiles more a tile.
 struct SeqTiles {
   int n_tiles;  // query tiles computed (the grid's max_seqlen cap applied)
   int n_full;   // full tiles among them
   int c16;
-  bool partial;  // tile n_tiles - 1 has fewer than 16 rows
+  int m;         // as SeqInfo::m
+  int rows;      // rows of a full tile
+  int q;         // as SeqInfo::q
+  bool partial;  // tile n_tiles - 1 has fewer than 16 * m rows
   int ng_full;   // column groups of a full tile
   bool full_narrow;  // a full tile is one column tile (G = 1): narrow chunks
   bool split;        // the sequence has partial rows (pbase >= 0): tiles may chunk
 };
 
 template <int CG, int W>
-__device__ __forceinline__ SeqTiles seq_tiles(const SeqInfo& s, int n_qtiles, int G) {
+__device__ __forceinline__ SeqTiles seq_tiles(const MixedParams& p, const SeqInfo& s) {
   SeqTiles t;
-  t.n_tiles = min((s.L + 15) >> 4, n_qtiles);
-  t.n_full = min(s.L >> 4, t.n_tiles);
+  t.m = s.m;
+  t.rows = s.m > 0 ? 16 * s.m : 16;
+  t.q = s.q;
   t.c16 = (s.c + 15) >> 4;
+  if (s.m > 0) {
+    const int rows = seq_rows(p, s.L);
+    t.n_full = rows / (16 * s.m);
+    t.n_tiles = t.n_full + (t.n_full * 16 * s.m < rows ? 1 : 0);
+    t.ng_full = 1;
+    t.full_narrow = false;
+  } else {
+    t.n_tiles = min((s.L + 15) >> 4, p.n_qtiles);
+    t.n_full = min(s.L >> 4, t.n_tiles);
+    t.ng_full = n_col_groups<CG>(p.G, seq_cg<CG>(s));
+    t.full_narrow = p.G <= 1;
+  }
   t.partial = t.n_tiles > t.n_full;
-  t.ng_full = n_col_groups<CG>(G, seq_cg<CG>(s));
-  t.full_narrow = G <= 1;
   t.split = s.pbase >= 0;
   return t;
 }
@@ -695,6 +781,12 @@ template <int W, class F>
 __device__ __forceinline__ void full_runs(const SeqTiles& st, F f) {
   if (!st.split) {
     if (st.n_full > 0) f(0, st.n_full - 1, 1);
+  } else if (st.m > 0) {
+    // full tile t has c16 + m * (t + 1) key tiles: those with more than q of
+    // them, from tile `lo` up, are two chunks
+    const int lo = min(st.n_full, st.q < st.c16 ? 0 : (st.q - st.c16) / st.m);
+    if (lo < st.n_full && f(lo, st.n_full - 1, 2)) return;
+    if (lo > 0) f(0, lo - 1, 1);
   } else if (st.full_narrow) chunk_runs<narrow_chunk_ktiles<W>()>(st.n_full, st.c16, f);
   else chunk_runs<wide_chunk_ktiles<W>()>(st.n_full, st.c16, f);
 }
@@ -718,7 +810,7 @@ __device__ __forceinline__ int tile_partial_off(const SeqTiles& st, int qt, int 
   int off = 0;
   full_runs<W>(st, [&](int lo, int hi, int k) {
     const int top = min(hi, below - 1);
-    if (k > 1 && top >= lo) off += (top - lo + 1) * 16 * H_q * k;
+    if (k > 1 && top >= lo) off += (top - lo + 1) * st.rows * H_q * k;
     return false;
   });
   return off;
@@ -728,14 +820,16 @@ __device__ __forceinline__ int tile_partial_off(const SeqTiles& st, int qt, int 
 // (the top tile's), the order in which batches of up to kRankSeqs sequences
 // deal their items; and its partial rows (P_b above: 0 if it does not split).
 template <int CG, int W>
-__device__ __forceinline__ int seq_items(const SeqInfo& s, const SeqTiles& st, int G, int H_q,
+__device__ __forceinline__ int seq_items(const MixedParams& p, const SeqInfo& s, const SeqTiles& st,
                                          int& weight, int& prows) {
+  const int H_q = p.H_q;
   int n = 0;
   weight = 0;
   prows = 0;
   if (st.n_tiles <= 0) return 0;
-  const TilePlan top = tile_plan<CG, W>(st.n_tiles - 1, s, G);
+  const TilePlan top = tile_plan<CG, W>(p, st.n_tiles - 1, s);
   weight = (top.n_ktiles + top.n_chunks - 1) / top.n_chunks;
+  if (s.m > 0) weight *= kWideWeight;
   if (st.n_tiles == 1 && top.n_ctiles == 1) {  // one narrow tile (a decode row)
     if (CIE_MIXED_NARROW_ORDER == 1) weight = 0;
     if (CIE_MIXED_NARROW_ORDER == 2) weight += 1 << 24;
@@ -747,7 +841,7 @@ __device__ __forceinline__ int seq_items(const SeqInfo& s, const SeqTiles& st, i
   const int ng = st.ng_full;
   full_runs<W>(st, [&](int lo, int hi, int k) {
     n += (hi - lo + 1) * ng * k;
-    if (k > 1) prows += (hi - lo + 1) * 16 * H_q * k;
+    if (k > 1) prows += (hi - lo + 1) * st.rows * H_q * k;
     return false;
   });
   return n;
@@ -756,12 +850,12 @@ __device__ __forceinline__ int seq_items(const SeqInfo& s, const SeqTiles& st, i
 // Item j of one sequence: its query tile and its index among the tile's
 // items (column group * chunks + chunk).
 template <int CG, int W>
-__device__ __forceinline__ void seq_locate(const SeqInfo& s, const SeqTiles& st, int G, int j,
-                                           int& qt, int& jt) {
+__device__ __forceinline__ void seq_locate(const MixedParams& p, const SeqInfo& s, const SeqTiles& st,
+                                           int j, int& qt, int& jt) {
   qt = st.n_tiles - 1;
   jt = j;
   if (st.partial) {
-    const TilePlan tp = tile_plan<CG, W>(st.n_tiles - 1, s, G);
+    const TilePlan tp = tile_plan<CG, W>(p, st.n_tiles - 1, s);
     const int np = tp.n_groups * tp.n_chunks;
     if (j < np) return;
     j -= np;
@@ -779,6 +873,27 @@ __device__ __forceinline__ void seq_locate(const SeqInfo& s, const SeqTiles& st,
     j -= cnt;
     return false;
   });
+}
+
+// Key tiles of a sequence's wide tiles, of one kv head.
+__device__ __forceinline__ float wide_ktiles(const MixedParams& p, const SeqInfo& s) {
+  if (s.m <= 0) return 0.f;
+  const int rows = seq_rows(p, s.L), r = 16 * s.m, n_full = rows / r;
+  float kt = (float)n_full * (float)((s.c + 15) >> 4) + 0.5f * (float)s.m * (float)n_full * (float)(n_full + 1);
+  if (n_full * r < rows) kt += (float)((s.c + rows + 15) >> 4);
+  return kt;
+}
+// SeqInfo::q from the batch's key tiles: kWideShare times the average
+// workgroup's share.  A workgroup streams a tile's keys alone, one step after
+// the other, so a tile far above the share would still run when the others'
+// work is done; its keys go to two workgroups (1,024 tokens over 8,000, 14 / 2
+// heads, D = 64: 164 us unsplit, 95; 4 x 2,048 on nothing: 87 split at once the
+// share, 75 at three times it; below 32 key tiles, 16 steps of ~0.7 us, the
+// parts' merge costs more than it saves).
+constexpr float kWideShare = 3.f;
+constexpr int kWideMinSplit = 32;
+__device__ __forceinline__ int wide_share(const MixedParams& p, float ktiles) {
+  return max(kWideMinSplit, (int)min(1e9f, kWideShare * ktiles * (float)p.H_kv / (float)p.wide_wg));
 }
 
 // Inclusive sum of (x, y) over the workgroup's first `span` threads (sm: NTH
@@ -816,7 +931,7 @@ __device__ __forceinline__ int prefix_search(const int* prefix, int n, int x) {
 
 // One work item: column group gi, chunk `chunk` of query tile qt of sequence
 // b, kv head g.
-template <int D, bool P32>
+template <int D, bool P32, bool kWide>
 __device__ __forceinline__ void process_item(const MixedParams& p, const SeqInfo& s, int b, int g,
                                              int qt, int j, f32x4* sm_facc, float2* sm_fml,
                                              f16x8* sm_q, int* sm_last, int item) {
@@ -827,13 +942,13 @@ __device__ __forceinline__ void process_item(const MixedParams& p, const SeqInfo
   const int wave = uniform(tid / kWave);
   const int r16 = lane & 15;
   const int grp = lane >> 4;
-  TilePlan tp = tile_plan<CG, W>(qt, s, p.G);
+  TilePlan tp = tile_plan<CG, W>(p, qt, s);
   // the block's base, taken once here, where the key loop's registers are
   // not yet live (after the loop, the run walk it takes spills scalars)
   if (tp.n_chunks > 1)
     tp.pblk = s.L <= 16 ? s.pbase  // one tile
-                        : uniform(s.pbase + tile_partial_off<CG, W>(seq_tiles<CG, W>(s, p.n_qtiles, p.G),
-                                                                    qt, p.H_q));
+                        : uniform(s.pbase +
+                                  tile_partial_off<CG, W>(seq_tiles<CG, W>(p, s), qt, p.H_q));
   const int gi = j / tp.n_chunks;
   const int chunk = j - gi * tp.n_chunks;
   const int ct0 = gi * tp.cg;
@@ -845,20 +960,34 @@ __device__ __forceinline__ void process_item(const MixedParams& p, const SeqInfo
   const PagedSrc src{p.k_pool,  p.v_pool,  p.block_table + s.slot * p.bt_stride,
                      (int64_t)g * p.pool_head_stride, p.pool_page_stride, p.n_pages,
                      p.page_size, p.err, p.tpp_magic, p.pool_bytes};
-  switch (n) {
+  const bool wide = kWide && s.m > 0;  // uniform
+  if (wide) {
+    f16* const sm = reinterpret_cast<f16*>(sm_facc);
+    __syncthreads();  // the previous item's fold may still be reading its slots
+    const int per = (tp.n_ctiles + kWideWaves - 1) / kWideWaves;  // column tiles a wave
+    if (per <= 1)
+      run_wide<D, 1>(p, s, tp, g, wave, chunk, kt0, kt1, src, r16, grp, sm);
+    else
+      run_wide<D, 2>(p, s, tp, g, 2 * wave, chunk, kt0, kt1, src, r16, grp, sm);
+  } else if constexpr (kWide) {  // one column tile (seq_blocks)
+    run_group<D, P32, 1>(p, s, tp, g, ct0, chunk, w0, w1, src, wave, r16, grp, sm_facc, sm_fml, sm_q,
+                         item);
+  } else {
+    switch (n) {
 #define CIE_GROUP_CASE(k)                                                                      \
   case k:                                                                                      \
     if constexpr (k <= CG)                                                                     \
       run_group<D, P32, k>(p, s, tp, g, ct0, chunk, w0, w1, src, wave, r16, grp, sm_facc,     \
                            sm_fml, sm_q, item);                                               \
     break;
-    CIE_GROUP_CASE(1)
-    CIE_GROUP_CASE(2)
-    CIE_GROUP_CASE(3)
-    CIE_GROUP_CASE(4)
+      CIE_GROUP_CASE(1)
+      CIE_GROUP_CASE(2)
+      CIE_GROUP_CASE(3)
+      CIE_GROUP_CASE(4)
 #undef CIE_GROUP_CASE
-    default:
-      break;
+      default:
+        break;
+    }
   }
   MIXED_TRACE(item, 2, __builtin_amdgcn_s_memrealtime());
   MIXED_TRACE(item, 5, (uint64_t)(tp.n_ctiles * 1000000 + tp.n_chunks * 10000 + (kt1 - kt0)));
@@ -875,7 +1004,14 @@ __device__ __forceinline__ void process_item(const MixedParams& p, const SeqInfo
   const int64_t n_words = (int64_t)p.B * p.H_kv * p.n_qtiles * kMaxColGroups;
   if (arrive_last(ctr, n_words, tp.n_chunks, sm_last, p.err)) {
     MIXED_TRACE(item, 4, __builtin_amdgcn_s_memrealtime());
-    merge_group<D>(p, s, tp, g, ct0, min(16 * n, tp.n_combos - 16 * ct0));
+    if (wide) {  // in blocks of column tiles that keep four units a thread
+      constexpr int kBlock = D <= 64 ? 4 : 2;
+      for (int c = 0; c < tp.n_ctiles; c += kBlock)
+        merge_group<D, kBlock>(p, s, tp, g, c, min(16 * kBlock, tp.n_combos - 16 * c));
+    } else {
+      merge_group<D, kWide ? 1 : col_group<D>()>(p, s, tp, g, ct0,
+                                                 min(16 * n, tp.n_combos - 16 * ct0));
+    }
     if (threadIdx.x == 0) counter_reset(ctr);
   }
   MIXED_TRACE(item, 3, __builtin_amdgcn_s_memrealtime());
@@ -890,24 +1026,29 @@ __device__ __forceinline__ void process_item(const MixedParams& p, const SeqInfo
 // (see the item loop), so no workgroup is launched for an empty slot.
 // Waves per SIMD the registers must allow: two when a wave carries at most
 // two column tiles or keeps its Q operands in LDS (D = 64), else one.
-template <int D>
+template <int D, bool kWide>
 constexpr int mixed_waves_per_simd() {
-  return D <= 64 && (col_group<D>() <= 2 || CIE_MIXED_QLDS) ? 2 : 1;
+  return kWide ? wide_waves_per_simd<D>() : D <= 64 && (col_group<D>() <= 2 || CIE_MIXED_QLDS) ? 2 : 1;
 }
 
 // The kernel's static LDS, element counts of its arrays: the waves' states
 // in the fold — [slot][d-tile][lane] (acc) and [slot][lane] (m, l), slot =
 // fold_slot(wave, column tile) — the item's Q operands, and the block scan.
-template <int D>
+template <int D, bool kWide>
 struct MixedLds {
   static constexpr int W = mixed_waves<D>();
-  static constexpr int kFold = col_group<D>() * (W - 1);
+  static constexpr int CG = kWide ? 1 : col_group<D>();
+  static constexpr int kFold = CG * (W - 1);
   static constexpr int facc = kFold * Geo<D>::NT * kWave;  // f32x4
   static constexpr int fml = kFold * kWave;                // float2
-  static constexpr int q = CIE_MIXED_QLDS ? col_group<D>() * Geo<D>::KS * kWave : 1;  // f16x8
+  static constexpr int q = CIE_MIXED_QLDS ? CG * Geo<D>::KS * kWave : 1;  // f16x8
+  // one array of 16-byte words holds the three, or (in a wide launch, whose
+  // items are of either kind) a wide item's K/V stages
+  static constexpr int fold_words = facc + (fml * sizeof(float2) + 15) / 16 + q;
+  static constexpr int stage_words = kWide ? WideLds<D>::bytes / 16 : 0;
+  static constexpr int words = fold_words > stage_words ? fold_words : stage_words;
   static constexpr int scan = W * kWave;                   // int2
-  static constexpr size_t bytes = facc * sizeof(f32x4) + fml * sizeof(float2) + q * sizeof(f16x8) +
-                                  scan * sizeof(int2) + 16 /* sm_last, aligned */;
+  static constexpr size_t bytes = words * 16 + scan * sizeof(int2) + 16 /* sm_last, aligned */;
 };
 // Every build must be able to plan a batch of kMaxSeqs sequences: its static
 // LDS plus the plan tables of kMaxSeqs sequences fit one workgroup's LDS.  (A
@@ -916,7 +1057,8 @@ struct MixedLds {
 // line of defence for devices with less.)
 template <int D>
 constexpr bool mixed_lds_fits() {
-  return MixedLds<D>::bytes + mixed_plan_lds(kMaxSeqs) <= kLdsPerWorkgroup;
+  return MixedLds<D, false>::bytes + mixed_plan_lds(kMaxSeqs) <= kLdsPerWorkgroup &&
+         MixedLds<D, true>::bytes + mixed_plan_lds(kMaxSeqs) <= kLdsPerWorkgroup;
 }
 
 // The batch's plan tables in LDS (sm_plan, mixed_plan_lds(B) bytes), all by
@@ -938,7 +1080,7 @@ struct PlanTables {
     order = prior + B;
     prefix = order + B;
   }
-  __device__ __forceinline__ SeqInfo seq(int pos) const {
+  __device__ __forceinline__ SeqInfo seq(const MixedParams& p, int pos, int wide_q) const {
     SeqInfo s;
     const int2 tb = tp[pos];
     s.t0 = uniform(tb.x);
@@ -946,6 +1088,8 @@ struct PlanTables {
     s.L = uniform(rows[pos]);
     s.c = uniform(prior[pos]);
     s.pbase = uniform(tb.y);
+    s.m = seq_blocks(p, s.L);
+    s.q = wide_q;
     return s;
   }
 };
@@ -955,7 +1099,8 @@ struct PlanTables {
 // per-sequence item counts, partial bases and the dealing order; returns
 // the item count (uniform).
 template <int D>
-__device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables& t, int2* sm_scan) {
+__device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables& t, int2* sm_scan,
+                                          int& wide_q) {
   constexpr int W = mixed_waves<D>();
   constexpr int NTH = W * kWave;
   constexpr int CG = col_group<D>();
@@ -973,14 +1118,16 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
     // wave), reading back only what it wrote itself — no barrier.
     const int lane = threadIdx.x & (kWave - 1);
     int n = 0, key = -1, prows = 0;
-    SeqInfo s{0, 0, 0, 0, 0};  // pbase 0: counted as split
+    SeqInfo s{0, 0, 0, 0, 0, 0, 0};  // pbase 0: counted as split
+    if (lane < B) s = seq_info(p, lane);
+    wide_q = p.wide_m > 0 ? uniform(wide_share(p, wave_sum(wide_ktiles(p, s)))) : 0;
+    s.q = wide_q;
     if (lane < B) {
-      s = seq_info(p, lane);
       if (blockIdx.x == 0 && threadIdx.x < kWave && ((s.L + 15) >> 4) > p.n_qtiles)
         set_err(p.err, CIE_ERRBIT_LEN);  // rows past max_seqlen are not computed
       int weight = 0;
       if (s.L > 0)
-        n = seq_items<CG, W>(s, seq_tiles<CG, W>(s, p.n_qtiles, p.G), p.G, p.H_q, weight, prows);
+        n = seq_items<CG, W>(p, s, seq_tiles<CG, W>(p, s), weight, prows);
       key = n > 0 ? weight : -1;
       prows = (int)min((int64_t)prows, p.part_cap + 1);
     }
@@ -1021,7 +1168,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
       s.pbase = (int64_t)pfx + prows <= p.part_cap ? pfx : -1;
       if (lane < B && s.pbase < 0 && s.L > 0) {
         int weight = 0, unused = 0;
-        n = seq_items<CG, W>(s, seq_tiles<CG, W>(s, p.n_qtiles, p.G), p.G, p.H_q, weight, unused);
+        n = seq_items<CG, W>(p, s, seq_tiles<CG, W>(p, s), weight, unused);
         key = n > 0 ? weight : -1;
       }
       rk = rank_key(key);
@@ -1054,8 +1201,23 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
     // tables, item counts and partial rows, sequences b = tid, tid + NTH,
     // ... (B <= kMaxSeqs), then a block scan of both: the item prefix and
     // each sequence's partial base.
+    wide_q = 0;
+    if (p.wide_m > 0) {
+      float kt = 0.f;
+      for (int b = threadIdx.x; b < B; b += NTH) kt += wide_ktiles(p, seq_info(p, b));
+      kt = wave_sum(kt);
+      float* const sm = reinterpret_cast<float*>(sm_scan);
+      if ((threadIdx.x & (kWave - 1)) == 0) sm[threadIdx.x / kWave] = kt;
+      __syncthreads();
+      kt = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; ++w) kt += sm[w];
+      wide_q = uniform(wide_share(p, kt));
+      __syncthreads();
+    }
     for (int b = threadIdx.x; b < B; b += NTH) {
-      const SeqInfo s = seq_info(p, b);  // pbase 0: counted as split
+      SeqInfo s = seq_info(p, b);  // pbase 0: counted as split
+      s.q = wide_q;
       sm_tp[b].x = (int)s.t0;
       sm_slot[b] = (int)s.slot;
       sm_rows[b] = s.L;
@@ -1064,7 +1226,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
         set_err(p.err, CIE_ERRBIT_LEN);  // rows past max_seqlen are not computed
       int n = 0, weight = 0, prows = 0;
       if (s.L > 0)
-        n = seq_items<CG, W>(s, seq_tiles<CG, W>(s, p.n_qtiles, p.G), p.G, p.H_q, weight, prows);
+        n = seq_items<CG, W>(p, s, seq_tiles<CG, W>(p, s), weight, prows);
       sm_prefix[b + 1] = n;
       sm_tp[b].y = (int)min((int64_t)prows, p.part_cap + 1);  // the base, after the scan
       sm_order[b] = b;
@@ -1096,14 +1258,16 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
         s.L = sm_rows[b];
         s.c = sm_prior[b];
         s.pbase = 0;
+        s.m = seq_blocks(p, s.L);
+        s.q = wide_q;
         int n = 0, weight = 0, prows = 0;
         if (s.L > 0)
-          n = seq_items<CG, W>(s, seq_tiles<CG, W>(s, p.n_qtiles, p.G), p.G, p.H_q, weight, prows);
+          n = seq_items<CG, W>(p, s, seq_tiles<CG, W>(p, s), weight, prows);
         const int pb = sm_tp[b].y;
         s.pbase = (int64_t)pb + min((int64_t)prows, p.part_cap + 1) <= p.part_cap ? pb : -1;
         sm_tp[b].y = s.pbase;
         if (s.pbase < 0 && s.L > 0)
-          n = seq_items<CG, W>(s, seq_tiles<CG, W>(s, p.n_qtiles, p.G), p.G, p.H_q, weight, prows);
+          n = seq_items<CG, W>(p, s, seq_tiles<CG, W>(p, s), weight, prows);
         sm_prefix[b + 1] = n;
       }
       __syncthreads();
@@ -1125,19 +1289,19 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
   return uniform(base);
 }
 
-template <int D, bool P32, bool kPlanned>
+template <int D, bool P32, bool kPlanned, bool kWide>
 __global__ __launch_bounds__(mixed_waves<D>() * kWave)
-__attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D>()))) void mixed_attention_kernel(
+__attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixed_attention_kernel(
     MixedParams p) {
   static_assert(col_group<D>() <= 4 && 8 / col_group<D>() <= kMaxColGroups, "column groups");
   static_assert(mixed_lds_fits<D>(),
                 "static LDS + the plan tables of kMaxSeqs sequences exceed a workgroup's LDS");
   constexpr int W = mixed_waves<D>();
   constexpr int NTH = W * kWave;
-  typedef MixedLds<D> Lds;
-  __shared__ f32x4 sm_facc[Lds::facc];
-  __shared__ float2 sm_fml[Lds::fml];
-  __shared__ f16x8 sm_q[Lds::q];
+  typedef MixedLds<D, kWide> Lds;
+  __shared__ f32x4 sm_facc[Lds::words];  // and behind it:
+  f16x8* const sm_q = reinterpret_cast<f16x8*>(sm_facc + Lds::facc);
+  float2* const sm_fml = reinterpret_cast<float2*>(sm_q + Lds::q);
   __shared__ int sm_last;
   // block scan (larger batches); a batch of up to 64 sequences ranks
   // through its first 2 * kWave words
@@ -1156,9 +1320,21 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D>()))) void mixed_atten
   const int g = blockIdx.x % p.H_kv;
   const int slot_r = blockIdx.x / p.H_kv;
   const int n_slots_r = gridDim.x / p.H_kv;  // workgroups per kv head
-  // item of round q for this workgroup (see the item loop)
-  auto item_of = [&](int q) { return q * n_slots_r + ((q & 1) ? n_slots_r - 1 - slot_r : slot_r); };
-  int n_items;
+  // Item of round q for this workgroup (see the item loop).  A wide launch has
+  // several workgroups a CU, workgroups w and w + CUs on the same one; at D = 64
+  // the rounds' direction alternates over CUs, so that a CU's workgroups do not
+  // all hold a sequence's longest tiles (4 x 2,048 tokens: 87 us a launch over
+  // workgroups, 75; D = 128, bound by the K/V stream, is slower that way: 312
+  // against 360 for 8,192 tokens of 16 / 4 heads).
+  constexpr int kPerCu = kWide && D <= 64 ? wide_waves_per_simd<D>() : 1;
+  const int n_cu_r = n_slots_r / kPerCu;
+  const int cu_r = kPerCu > 1 ? slot_r % n_cu_r : slot_r;
+  const int layer = kPerCu > 1 ? slot_r / n_cu_r : 0;
+  auto item_of = [&](int q) {
+    const int r = q * kPerCu + layer;
+    return r * n_cu_r + ((r & 1) ? n_cu_r - 1 - cu_r : cu_r);
+  };
+  int n_items, wide_q;
   if constexpr (kPlanned) {
     // The step's plan: a header, then one 8-word descriptor per item.  The
     // header and the descriptors of this workgroup's first kDescRounds
@@ -1175,14 +1351,16 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D>()))) void mixed_atten
     const int4 h1 = *reinterpret_cast<const int4*>(hdr + 4);
     __syncthreads();
     n_items = uniform(h0.x);
+    wide_q = uniform(h1.w);
     // a plan made for another batch shape, budget or partial layout
     if (uniform(h0.y) != (int)p.part_cap || uniform(h0.z) != p.B || uniform(h0.w) != p.n_qtiles ||
-        uniform(h1.x) != p.H_q || uniform(h1.y) != p.H_kv || n_items > p.plan_cap) {
+        uniform(h1.x) != p.H_q || uniform(h1.y) != p.H_kv || uniform(h1.z) != p.wide_m ||
+        n_items > p.plan_cap) {
       if (blockIdx.x == 0 && threadIdx.x == 0) set_err(p.err, CIE_ERRBIT_PLAN);
       return;
     }
   } else {
-    n_items = plan_batch<D>(p, tables, sm_scan);
+    n_items = plan_batch<D>(p, tables, sm_scan, wide_q);
   }
   MIXED_TRACE(0, 6, __builtin_amdgcn_s_memrealtime());  // planning done
   MIXED_TRACE(0, 14, (uint64_t)blockIdx.x);
@@ -1214,16 +1392,18 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D>()))) void mixed_atten
       s.L = uniform(d1.y);
       s.c = uniform(d1.z);
       s.pbase = uniform(d1.w);
+      s.m = seq_blocks(p, s.L);
+      s.q = wide_q;
     } else {
       const int pos = prefix_search(tables.prefix, p.B, item);
       b = uniform(tables.order[pos]);
       const int j = item - uniform(tables.prefix[pos]);
-      s = tables.seq(pos);
-      seq_locate<CG, W>(s, seq_tiles<CG, W>(s, p.n_qtiles, p.G), p.G, j, qt, jt);
+      s = tables.seq(p, pos, wide_q);
+      seq_locate<CG, W>(p, s, seq_tiles<CG, W>(p, s), j, qt, jt);
     }
     MIXED_TRACE(item, 1, __builtin_amdgcn_s_memrealtime());
     MIXED_TRACE(item, 7, (uint64_t)(b * 1000 + qt));
-    process_item<D, P32>(p, s, b, g, uniform(qt), uniform(jt), sm_facc, sm_fml, sm_q, &sm_last,
+    process_item<D, P32, kWide>(p, s, b, g, uniform(qt), uniform(jt), sm_facc, sm_fml, sm_q, &sm_last,
                          item);
   }
 }
@@ -1232,18 +1412,19 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D>()))) void mixed_atten
 // A step's plan for its planned mixed launches (cie_mixed_plan): one
 // workgroup plans the batch as every workgroup of an unplanned launch does,
 // then writes the header {items, partial budget (rows), B, query tiles,
-// H_q, H_kv, 0, 0} and, per item in dealing order, its descriptor
+// H_q, H_kv, wide_m, wide_q} and, per item in dealing order, its descriptor
 // {b, query tile, index in tile, t0, slot, rows, prior, partial base}.
 template <int D>
 __global__ __launch_bounds__(mixed_waves<D>() * kWave) void mixed_plan_kernel(MixedParams p) {
   constexpr int W = mixed_waves<D>();
   constexpr int NTH = W * kWave;
   constexpr int CG = col_group<D>();
-  typedef MixedLds<D> Lds;
+  typedef MixedLds<D, false> Lds;
   __shared__ __attribute__((aligned(16))) int2 sm_scan[Lds::scan];
   extern __shared__ __attribute__((aligned(16))) char sm_plan[];
   const PlanTables t(sm_plan, p.B);
-  const int n_items = plan_batch<D>(p, t, sm_scan);
+  int wide_q;
+  const int n_items = plan_batch<D>(p, t, sm_scan, wide_q);
   __syncthreads();
   int32_t* const out = p.plan_out;
   const bool fits = n_items <= p.plan_cap;
@@ -1252,7 +1433,7 @@ __global__ __launch_bounds__(mixed_waves<D>() * kWave) void mixed_plan_kernel(Mi
     // sequences can exceed it) gets an empty plan and CIE_ERRBIT_PLAN
     if (!fits) set_err(p.err, CIE_ERRBIT_PLAN);
     *reinterpret_cast<int4*>(out) = int4{fits ? n_items : 0, (int)p.part_cap, p.B, p.n_qtiles};
-    *reinterpret_cast<int4*>(out + 4) = int4{p.H_q, p.H_kv, 0, 0};
+    *reinterpret_cast<int4*>(out + 4) = int4{p.H_q, p.H_kv, p.wide_m, wide_q};
   }
   if (!fits) return;
   for (int i = threadIdx.x; i < n_items; i += NTH) {
@@ -1270,23 +1451,24 @@ __global__ __launch_bounds__(mixed_waves<D>() * kWave) void mixed_plan_kernel(Mi
     s.L = t.rows[lo];
     s.c = t.prior[lo];
     s.pbase = tb.y;
+    s.m = seq_blocks(p, s.L);
+    s.q = wide_q;
     int qt, jt;
-    seq_locate<CG, W>(s, seq_tiles<CG, W>(s, p.n_qtiles, p.G), p.G, i - t.prefix[lo], qt, jt);
+    seq_locate<CG, W>(p, s, seq_tiles<CG, W>(p, s), i - t.prefix[lo], qt, jt);
     int32_t* const d = out + kPlanHeader + (int64_t)i * 8;
     *reinterpret_cast<int4*>(d) = int4{t.order[lo], qt, jt, (int)s.t0};
     *reinterpret_cast<int4*>(d + 4) = int4{(int)s.slot, s.L, s.c, s.pbase};
   }
 }
 
-// Workgroups of the mixed grid: CIE_MIXED_WG_PER_CU per CU, a whole number
-// per kv head.
-static int mixed_workgroups(int H_kv) {
+// Workgroups of the mixed grid: a whole number per kv head.
+static int mixed_workgroups(int H_kv, int per_cu) {
   int dev = 0, n_cu = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
-  int per_head = n_cu * CIE_MIXED_WG_PER_CU / H_kv;
+  int per_head = n_cu / H_kv;
   if (per_head < 1) per_head = 1;
-  return per_head * H_kv;
+  return per_head * H_kv * per_cu;
 }
 
 // LDS a workgroup may use on the current device (160 KiB on gfx950).
@@ -1312,31 +1494,28 @@ static int64_t static_lds_of(K kernel) {
              : 0;
 }
 
-template <int D, bool P32, bool kPlanned>
-static int64_t mixed_static_lds() {
-  static int64_t bytes = -1;
-  if (bytes < 0) bytes = static_lds_of(mixed_attention_kernel<D, P32, kPlanned>);
-  return bytes;
-}
-
-template <int D, bool kPlanned>
-static int launch_mixed(const MixedParams& p, hipStream_t stream) {
-  dim3 grid(mixed_workgroups(p.H_kv), 1, 1);
+template <int D, bool P32, bool kPlanned, bool kWide>
+static int launch_mixed_kernel(const MixedParams& p, hipStream_t stream) {
+  static int64_t lds = -1;
+  if (lds < 0) lds = static_lds_of(mixed_attention_kernel<D, P32, kPlanned, kWide>);
+  dim3 grid(kWide ? p.wide_wg : mixed_workgroups(p.H_kv, CIE_MIXED_WG_PER_CU), 1, 1);
   // a batch whose plan tables would take the workgroup past the device's
   // LDS is refused here (the dispatch itself would be rejected); a planned
   // launch reads its plan instead of building the tables
   const size_t dyn = kPlanned ? 0 : mixed_plan_lds(p.B);
-  const int64_t lds = (p.pool_bytes != 0 ? mixed_static_lds<D, true, kPlanned>()
-                                         : mixed_static_lds<D, false, kPlanned>()) +
-                      (int64_t)dyn;
-  if (lds > device_lds_limit()) return CIE_EUNSUPPORTED;
-  if (p.pool_bytes != 0)
-    hipLaunchKernelGGL((mixed_attention_kernel<D, true, kPlanned>), grid,
-                       dim3(mixed_waves<D>() * kWave), dyn, stream, p);
-  else
-    hipLaunchKernelGGL((mixed_attention_kernel<D, false, kPlanned>), grid,
-                       dim3(mixed_waves<D>() * kWave), dyn, stream, p);
+  if (lds + (int64_t)dyn > device_lds_limit()) return CIE_EUNSUPPORTED;
+  hipLaunchKernelGGL((mixed_attention_kernel<D, P32, kPlanned, kWide>), grid,
+                     dim3(mixed_waves<D>() * kWave), dyn, stream, p);
   return (int)hipGetLastError();
+}
+
+template <int D, bool kPlanned>
+static int launch_mixed(const MixedParams& p, hipStream_t stream) {
+  if (p.wide_m > 0)
+    return p.pool_bytes != 0 ? launch_mixed_kernel<D, true, kPlanned, true>(p, stream)
+                             : launch_mixed_kernel<D, false, kPlanned, true>(p, stream);
+  return p.pool_bytes != 0 ? launch_mixed_kernel<D, true, kPlanned, false>(p, stream)
+                           : launch_mixed_kernel<D, false, kPlanned, false>(p, stream);
 }
 
 template <int D>
@@ -1391,7 +1570,9 @@ extern "C" int64_t cie_mixed_partials_bytes(int64_t total_T, int64_t H_q, int64_
   const int64_t chunked = kMaxChunks * (total_T < kDefaultChunkedTokens ? total_T : kDefaultChunkedTokens);
   int64_t rows = (per_token > chunked ? per_token : chunked) * H_q;
   if (rows > kMaxPartRows) rows = kMaxPartRows;
-  return mixed_layout(rows, D).total;
+  // (the alignment of the layout's regions, which mixed_partial_rows takes off,
+  // on top: a batch that needs exactly these rows fits)
+  return rows * 4 * (D + 2) + 3 * 256;
 }
 
 extern "C" int64_t cie_mixed_counters(int64_t B, int64_t H_kv, int64_t max_seqlen) {
@@ -1408,6 +1589,25 @@ extern "C" int cie_mixed_trace_buffer(void* buf) {
   return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_mixed_trace), &p, sizeof(p));
 }
 #endif
+
+// Whether a launch is wide (see wide_tiles.h), from the number of wide tiles
+// that total_T rows make if they are all prefill: enough of them must fill the
+// chip, as a wide tile runs a longer serial loop than a narrow one.  The line
+// lies lower where narrow items share their keys among fewer columns: a narrow
+// item holds 4 column tiles at D = 64 (G at most, for G < 4), 1 at D = 128.
+// Measured, us a launch narrow / wide, at a line's two sides: D = 64, 14 / 2
+// heads: 256 tiles (2,048 tokens on nothing) 33 / 38, 512 (4,096) 89 / 86, 1,024
+// (28 / 4 heads) 159 / 106; 8 / 8 heads: 64 tiles 22 / 28, 128 (2,048 tokens)
+// 54 / 39; D = 128, 14 / 2 heads: 64 tiles (512 tokens) 22 / 27, 128 43 / 38, 512
+// 359 / 133.
+static void wide_rule(MixedParams& p, int64_t D) {
+  const int m = kWideColTiles / p.G;  // (G <= 8)
+  const int64_t tiles = p.total_T * p.H_kv / (16 * m);
+  const int64_t enough = D <= 64 ? 128 * (p.G < 4 ? p.G : 4) : 96;
+  if (tiles < enough) return;
+  p.wide_m = m;
+  p.wide_wg = mixed_workgroups(p.H_kv, D <= 64 ? wide_waves_per_simd<64>() : wide_waves_per_simd<128>());
+}
 
 // Checks of the batch shape shared by the entry points, and the parameters
 // they determine (the budget of partial rows from partials_bytes included).
@@ -1445,6 +1645,7 @@ static int mixed_shape(MixedParams& p, int64_t B, int64_t total_T, int64_t max_s
   // The buffer sets the budget of partial rows: sequences whose split tiles
   // do not fit run unsplit (the plan's pbase).
   p.part_cap = mixed_partial_rows(partials_bytes, D);
+  wide_rule(p, D);
   return CIE_OK;
 }
 

@@ -1,0 +1,113 @@
+"""Wide launches of the mixed kernel (enough prefill rows to fill the chip) against the oracle.
+
+Each case is sized past the rule that makes a launch wide — tiles of
+16 * floor(8 / G) rows times kv heads, at least 96 at D = 128 and 128 * min(G, 4)
+at D = 64 — and compared with the fp32 oracle, planned and unplanned (which
+must agree bit for bit), at the edges of the tiles: lengths of a whole tile,
+one row more and less, chunks of one and two column tiles a wave, sequences
+that split their keys and decode rows beside them."""
+import pytest
+import torch
+
+from custom_inference_engine_amd import kv_append_tokens, mixed_gqa_attention, mixed_plan
+from oracle import inputs
+from tests.conftest import assert_attn_close
+from tests.gpu_helpers import DEV, bits, err_word, note, oracle_mixed
+
+pytestmark = pytest.mark.gpu
+
+
+def _wide(case, h_q, h_kv, d):
+    rows = 16 * (8 // (h_q // h_kv))
+    tiles = case.T * h_kv // rows
+    return tiles >= (96 if d == 128 else 128 * min(4, h_q // h_kv))
+
+
+def _run(case, h_q, max_seqlen=None, poison=False, rows=slice(None)):
+    c = case.to(DEV)
+    kp, vp = c.k_pool.clone(), c.v_pool.clone()
+    if poison:  # pool rows past each sequence's end hold NaN (as uninitialised memory may)
+        used = torch.zeros(kp.shape[0], kp.shape[2], dtype=torch.bool)
+        for b in range(case.B):
+            n = int(case.kv_lens[b] + case.new_lens[b])
+            pg = case.block_table[int(case.slot_ids[b])]
+            pos = torch.arange(n)
+            used[pg[pos // case.page_size], pos % case.page_size] = True
+        kp.transpose(1, 2)[~used.to(DEV)] = float("nan")
+        vp.transpose(1, 2)[~used.to(DEV)] = float("nan")
+    err = err_word()
+    kv_append_tokens(kp, vp, c.k_new, c.v_new, c.pages, c.offsets, err=err)
+    ms = max_seqlen or int(case.new_lens.max())
+    plan = mixed_plan(kp, c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table, ms, case.T, h_q, err=err)
+    o = [mixed_gqa_attention(c.q, kp, vp, ms, c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table, err=err,
+                             plan=p) for p in (plan, None)]
+    torch.cuda.synchronize()
+    # (rows that are not computed hold what torch.empty_like left there)
+    assert torch.equal(bits(o[0][0, rows]), bits(o[1][0, rows])), "planned and unplanned differ"
+    return o[0][0].float().cpu(), int(err.item())
+
+
+CASES = {
+    # h_q, h_kv, d, page_size, prior, new
+    "d128": (14, 2, 128, 16, [0, 700, 33, 0, 5, 90, 3000], [320, 17, 250, 16, 1, 1, 200]),
+    "d128-g4-ps32": (32, 8, 128, 32, [0, 1000, 40, 7], [31, 1, 33, 400]),
+    "d128-g1": (8, 8, 128, 16, [0, 500, 0], [127, 1, 1500]),
+    "d128-g8": (16, 2, 128, 16, [100, 2], [700, 300]),
+    "d64-g1": (8, 8, 64, 16, [0, 3, 200, 64], [900, 129, 1100, 16]),
+    "d64-g2": (8, 4, 64, 32, [0, 31, 1500], [2000, 65, 2200]),
+    "d64-g7": (14, 2, 64, 16, [0, 15, 600, 40, 1000], [2100, 15, 1990, 1, 1]),
+    "d64-g5": (20, 4, 64, 16, [10, 0], [17, 2200]),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_wide_launch_matches_the_oracle(native_lib, name):
+    h_q, h_kv, d, ps, prior, new = CASES[name]
+    case = inputs.make_case(prior, new, h_q=h_q, h_kv=h_kv, d=d, page_size=ps, seed=91)
+    assert _wide(case, h_q, h_kv, d)
+    note(f"wide {name}")
+    o, err = _run(case, h_q, poison=True)
+    assert err == 0
+    want, written = oracle_mixed(case)
+    assert_attn_close(o[written], want[written], what=name)
+
+
+def test_wide_launch_splits_long_tiles(native_lib):
+    """One long chunk over a long prefix beside short ones: its tiles are far above
+    the average share of keys and split in two; with no partials budget the same
+    tiles run whole, and both match the oracle."""
+    case = inputs.make_case([6000, 0, 0], [300, 200, 300], d=128, seed=92)
+    assert _wide(case, 14, 2, 128)
+    note("wide split")
+    o, err = _run(case, 14)
+    assert err == 0
+    want, written = oracle_mixed(case)
+    assert_attn_close(o[written], want[written], what="split")
+    c = case.to(DEV)
+    kp, vp = (t.to(DEV) for t in case.appended_pools())
+    whole = mixed_gqa_attention(c.q, kp, vp, 300, c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table,
+                                partials_bytes=0)
+    assert_attn_close(whole[0].float().cpu()[written], want[written], what="whole")
+
+
+def test_wide_launch_of_many_sequences(native_lib):
+    """More than 64 sequences (the block plan), most of them decode rows."""
+    new = [1 if i % 3 else 29 for i in range(100)]
+    case = inputs.make_case([(i * 37) % 400 for i in range(100)], new, d=128, seed=93)
+    assert _wide(case, 14, 2, 128)
+    note("wide block plan")
+    o, err = _run(case, 14)
+    assert err == 0
+    want, written = oracle_mixed(case)
+    assert_attn_close(o[written], want[written], what="many")
+
+
+def test_wide_launch_past_max_seqlen(native_lib):
+    """Rows past max_seqlen (rounded up to 16) are reported and not computed, the others are."""
+    case = inputs.make_case([0, 100], [500, 500], d=128, seed=94)
+    note("wide max_seqlen")
+    rows = torch.cat([torch.arange(208), 500 + torch.arange(208)])
+    o, err = _run(case, 14, max_seqlen=200, rows=rows)
+    assert err == 2  # CIE_ERRBIT_LEN
+    want, _ = oracle_mixed(case)
+    assert_attn_close(o[rows], want[rows], what="max_seqlen")
