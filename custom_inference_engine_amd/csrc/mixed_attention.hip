@@ -105,6 +105,7 @@ namespace cie {
 
 constexpr int kWavePairs = CIE_MIXED_WAVE_PAIRS;
 constexpr int kMaxChunks = 16;    // workgroups per (tile, column group) at most
+constexpr int kWideMaxChunks = 8;  // the same of a wide tile
 constexpr int kWideWeight = 3;    // cost of a wide item's key tile, in a narrow item's
 constexpr int kMaxColGroups = 8;  // column groups per tile at most (<= 8 column tiles)
 // Partial rows a launch uses at most, whatever the buffer: with each
@@ -188,7 +189,7 @@ struct SeqInfo {
   // not split (the batch's partial rows would exceed the caller's buffer)
   int pbase;
   int m;  // wide query tiles: their 16-row blocks (seq_blocks); 0: tiles of 16 rows
-  int q;  // wide query tiles of more key tiles than this are two chunks (wide_share)
+  int q;  // key tiles a chunk of a wide query tile holds (wide_share)
 };
 
 // In a wide launch every sequence of more than one column tile is cut into
@@ -274,7 +275,7 @@ __device__ __forceinline__ TilePlan tile_plan(const MixedParams& p, int qt, cons
   t.n_pairs = (t.n_ktiles + 1) >> 1;
   constexpr int kPerNarrow = W * CIE_MIXED_NARROW_PAIRS;
   constexpr int kPerWide = W * kWavePairs;
-  const int chunks = wide ? (t.n_ktiles > s.q ? 2 : 1)
+  const int chunks = wide ? min(kWideMaxChunks, (t.n_ktiles + s.q - 1) / s.q)
                      : t.n_ctiles == 1 ? (t.n_pairs + kPerNarrow - 1) / kPerNarrow
                                        : (t.n_pairs + kPerWide - 1) / kPerWide;
   t.n_chunks = s.pbase < 0 ? 1 : max(1, min(kMaxChunks, chunks));
@@ -782,11 +783,15 @@ __device__ __forceinline__ void full_runs(const SeqTiles& st, F f) {
   if (!st.split) {
     if (st.n_full > 0) f(0, st.n_full - 1, 1);
   } else if (st.m > 0) {
-    // full tile t has c16 + m * (t + 1) key tiles: those with more than q of
-    // them, from tile `lo` up, are two chunks
-    const int lo = min(st.n_full, st.q < st.c16 ? 0 : (st.q - st.c16) / st.m);
-    if (lo < st.n_full && f(lo, st.n_full - 1, 2)) return;
-    if (lo > 0) f(0, lo - 1, 1);
+    // full tile t has c16 + m * (t + 1) key tiles, q a chunk
+    for (int t_hi = st.n_full - 1; t_hi >= 0;) {
+      const int k = min(kWideMaxChunks, (st.c16 + st.m * (t_hi + 1) + st.q - 1) / st.q);
+      // lowest tile with the same (clamped) count: more than (k - 1) * q key tiles
+      const int past = (k - 1) * st.q - st.c16;
+      const int t_lo = past > 0 ? past / st.m : 0;
+      if (f(t_lo, t_hi, k)) return;
+      t_hi = t_lo - 1;
+    }
   } else if (st.full_narrow) chunk_runs<narrow_chunk_ktiles<W>()>(st.n_full, st.c16, f);
   else chunk_runs<wide_chunk_ktiles<W>()>(st.n_full, st.c16, f);
 }
@@ -875,25 +880,45 @@ __device__ __forceinline__ void seq_locate(const MixedParams& p, const SeqInfo& 
   });
 }
 
-// Key tiles of a sequence's wide tiles, of one kv head.
-__device__ __forceinline__ float wide_ktiles(const MixedParams& p, const SeqInfo& s) {
-  if (s.m <= 0) return 0.f;
+// Wide tiles of a sequence and their key tiles, of one kv head.
+struct WideWork {
+  float tiles, ktiles;
+};
+__device__ __forceinline__ WideWork wide_work(const MixedParams& p, const SeqInfo& s) {
+  if (s.m <= 0) return {0.f, 0.f};
   const int rows = seq_rows(p, s.L), r = 16 * s.m, n_full = rows / r;
-  float kt = (float)n_full * (float)((s.c + 15) >> 4) + 0.5f * (float)s.m * (float)n_full * (float)(n_full + 1);
-  if (n_full * r < rows) kt += (float)((s.c + rows + 15) >> 4);
-  return kt;
+  WideWork w{(float)n_full,
+             (float)n_full * (float)((s.c + 15) >> 4) + 0.5f * (float)s.m * (float)n_full * (float)(n_full + 1)};
+  if (n_full * r < rows) {
+    w.tiles += 1.f;
+    w.ktiles += (float)((s.c + rows + 15) >> 4);
+  }
+  return w;
 }
-// SeqInfo::q from the batch's key tiles: kWideShare times the average
-// workgroup's share.  A workgroup streams a tile's keys alone, one step after
-// the other, so a tile far above the share would still run when the others'
-// work is done; its keys go to two workgroups (1,024 tokens over 8,000, 14 / 2
-// heads, D = 64: 164 us unsplit, 95; 4 x 2,048 on nothing: 87 split at once the
-// share, 75 at three times it; below 32 key tiles, 16 steps of ~0.7 us, the
-// parts' merge costs more than it saves).
-constexpr float kWideShare = 3.f;
-constexpr int kWideMinSplit = 32;
-__device__ __forceinline__ int wide_share(const MixedParams& p, float ktiles) {
-  return max(kWideMinSplit, (int)min(1e9f, kWideShare * ktiles * (float)p.H_kv / (float)p.wide_wg));
+// SeqInfo::q from the batch's wide tiles: a multiple of the average workgroup's
+// share of their key tiles.  A workgroup streams a tile's keys alone, one step
+// after the other, so a tile far above the share would still run when the
+// others' work is done; its keys go to several workgroups, at the price of
+// partials and a merge.  Few tiles for the chip (long prefixes under few rows)
+// split to 1.5 times the share, as many tiles as workgroups or more to 3 times
+// it, where the other tiles fill the gaps.  Measured, us a call with at most two
+// chunks of 3 times the share / so: D = 128: 1,536 tokens over 8,000 (14 / 2
+// heads) 257 / 175, 3 x 512 over 4,000 130 / 100, 768 over 8,000 134 / 100;
+// D = 64, 8 / 8 heads: 2,048 over 8,000 108 / 88; 4 x 2,048 on nothing (14 / 2)
+// 72 / 68.  Chunks of fewer than 16 steps (D = 128: 24) cost more in the merge
+// than they save (1,024 over 2,000: 75 us at 16 steps, 61 at 32).
+constexpr float kWideShareMin = 1.5f, kWideShareMax = 3.f, kWideShareSlope = 6.f;
+template <int D>
+constexpr int kWideMinSplit = D <= 64 ? 32 : 48;
+template <int D>
+__device__ __forceinline__ int wide_share(const MixedParams& p, WideWork w) {
+  const float per_wg = (float)p.H_kv / (float)p.wide_wg;
+  float q = fminf(kWideShareMax, fmaxf(kWideShareMin, kWideShareSlope * w.tiles * per_wg)) * w.ktiles * per_wg;
+  // a batch of n tiles has fewer than n + ktiles / q chunks: kept to three
+  // quarters of the partials budget (the rest is for split decode rows)
+  const float chunks = 0.75f * (float)p.part_cap / (float)(16 * p.wide_m * p.H_q) - w.tiles;
+  if (q * chunks < w.ktiles) q = chunks > 0.f ? fminf(1e9f, w.ktiles / chunks) : 1e9f;
+  return max(kWideMinSplit<D>, (int)fminf(1e9f, q));
 }
 
 // Inclusive sum of (x, y) over the workgroup's first `span` threads (sm: NTH
@@ -1120,7 +1145,11 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
     int n = 0, key = -1, prows = 0;
     SeqInfo s{0, 0, 0, 0, 0, 0, 0};  // pbase 0: counted as split
     if (lane < B) s = seq_info(p, lane);
-    wide_q = p.wide_m > 0 ? uniform(wide_share(p, wave_sum(wide_ktiles(p, s)))) : 0;
+    wide_q = 0;
+    if (p.wide_m > 0) {
+      const WideWork w = wide_work(p, s);
+      wide_q = uniform(wide_share<D>(p, {wave_sum(w.tiles), wave_sum(w.ktiles)}));
+    }
     s.q = wide_q;
     if (lane < B) {
       if (blockIdx.x == 0 && threadIdx.x < kWave && ((s.L + 15) >> 4) > p.n_qtiles)
@@ -1203,16 +1232,23 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
     // each sequence's partial base.
     wide_q = 0;
     if (p.wide_m > 0) {
-      float kt = 0.f;
-      for (int b = threadIdx.x; b < B; b += NTH) kt += wide_ktiles(p, seq_info(p, b));
-      kt = wave_sum(kt);
-      float* const sm = reinterpret_cast<float*>(sm_scan);
-      if ((threadIdx.x & (kWave - 1)) == 0) sm[threadIdx.x / kWave] = kt;
+      WideWork w{0.f, 0.f};
+      for (int b = threadIdx.x; b < B; b += NTH) {
+        const WideWork x = wide_work(p, seq_info(p, b));
+        w.tiles += x.tiles;
+        w.ktiles += x.ktiles;
+      }
+      w = {wave_sum(w.tiles), wave_sum(w.ktiles)};
+      float2* const sm = reinterpret_cast<float2*>(sm_scan);
+      if ((threadIdx.x & (kWave - 1)) == 0) sm[threadIdx.x / kWave] = float2{w.tiles, w.ktiles};
       __syncthreads();
-      kt = 0.f;
+      w = {0.f, 0.f};
 #pragma unroll
-      for (int w = 0; w < W; ++w) kt += sm[w];
-      wide_q = uniform(wide_share(p, kt));
+      for (int i = 0; i < W; ++i) {
+        w.tiles += sm[i].x;
+        w.ktiles += sm[i].y;
+      }
+      wide_q = uniform(wide_share<D>(p, w));
       __syncthreads();
     }
     for (int b = threadIdx.x; b < B; b += NTH) {
@@ -1315,6 +1351,10 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
   __shared__ __attribute__((aligned(16))) int4 sm_desc[kPlanned ? 2 * kDescRounds : 1];
   const PlanTables tables(sm_plan, p.B);
 
+  // (known to the compiler: no item of a narrow launch is wide.  A division by
+  // the wide chunk length, taken per item ahead of the test, cost 2 %)
+  if constexpr (!kWide) p.wide_m = 0;
+
   constexpr int CG = col_group<D>();
   MIXED_TRACE(0, 15, __builtin_amdgcn_s_memrealtime());  // workgroup start
   const int g = blockIdx.x % p.H_kv;
@@ -1351,7 +1391,7 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
     const int4 h1 = *reinterpret_cast<const int4*>(hdr + 4);
     __syncthreads();
     n_items = uniform(h0.x);
-    wide_q = uniform(h1.w);
+    wide_q = max(1, uniform(h1.w));
     // a plan made for another batch shape, budget or partial layout
     if (uniform(h0.y) != (int)p.part_cap || uniform(h0.z) != p.B || uniform(h0.w) != p.n_qtiles ||
         uniform(h1.x) != p.H_q || uniform(h1.y) != p.H_kv || uniform(h1.z) != p.wide_m ||
@@ -1559,6 +1599,17 @@ static int64_t mixed_partial_rows(int64_t bytes, int64_t D) {
 // prefill: 101.8 us at 2 rows per token, 56.9 at 16).
 constexpr int64_t kDefaultRowsPerToken = 2;
 constexpr int64_t kDefaultChunkedTokens = 64;
+// Wide tiles (from the smallest launches that have them: wide_rule) split up to
+// kWideMaxChunks times where a few hundred rows attend thousands of keys: 8 rows
+// for each of the first 2,048 tokens (D = 128, its rows twice as long: 1,024;
+// 136 MB at 32 heads).  512 tokens over 8,000 keys (14 / 2 heads, D = 128): 163 us
+// unsplit, as 2 rows per token leave it, 91 at 8; 2,048 over 8,000 (8 / 8 heads,
+// D = 64) 117 us with 4 rows, which make three uneven chunks a tile of two.
+constexpr int64_t kDefaultWideRowsPerToken = 8;
+static int64_t default_wide_rows(int64_t total_T, int64_t D) {
+  const int64_t from = D <= 64 ? 1100 : 128, most = D <= 64 ? 2048 : 1024;
+  return total_T < from ? 0 : kDefaultWideRowsPerToken * (total_T < most ? total_T : most);
+}
 
 }  // namespace cie
 
@@ -1567,12 +1618,14 @@ using namespace cie;
 extern "C" int64_t cie_mixed_partials_bytes(int64_t total_T, int64_t H_q, int64_t D) {
   if (total_T < 0 || H_q <= 0 || D <= 0 || total_T > ((int64_t)1 << 40) / H_q) return -1;
   const int64_t per_token = kDefaultRowsPerToken * total_T;
+  const int64_t wide = default_wide_rows(total_T, D);
   const int64_t chunked = kMaxChunks * (total_T < kDefaultChunkedTokens ? total_T : kDefaultChunkedTokens);
-  int64_t rows = (per_token > chunked ? per_token : chunked) * H_q;
+  int64_t rows = (per_token > chunked ? per_token : chunked);
+  rows = (rows > wide ? rows : wide) * H_q;
   if (rows > kMaxPartRows) rows = kMaxPartRows;
-  // (the alignment of the layout's regions, which mixed_partial_rows takes off,
-  // on top: a batch that needs exactly these rows fits)
-  return rows * 4 * (D + 2) + 3 * 256;
+  // (a multiple of 256, and the alignment of the layout's regions, which
+  // mixed_partial_rows takes off, on top: a batch of exactly these rows fits)
+  return (rows * 4 * (D + 2) + 255) / 256 * 256 + 3 * 256;
 }
 
 extern "C" int64_t cie_mixed_counters(int64_t B, int64_t H_kv, int64_t max_seqlen) {
@@ -1595,16 +1648,22 @@ extern "C" int cie_mixed_trace_buffer(void* buf) {
 // chip, as a wide tile runs a longer serial loop than a narrow one.  The line
 // lies lower where narrow items share their keys among fewer columns: a narrow
 // item holds 4 column tiles at D = 64 (G at most, for G < 4), 1 at D = 128.
-// Measured, us a launch narrow / wide, at a line's two sides: D = 64, 14 / 2
-// heads: 256 tiles (2,048 tokens on nothing) 33 / 38, 512 (4,096) 89 / 86, 1,024
-// (28 / 4 heads) 159 / 106; 8 / 8 heads: 64 tiles 22 / 28, 128 (2,048 tokens)
-// 54 / 39; D = 128, 14 / 2 heads: 64 tiles (512 tokens) 22 / 27, 128 43 / 38, 512
-// 359 / 133.
+// Measured, us a call with its append, narrow / wide, below a line and past it,
+// one prompt of n tokens on nothing first, the same over 2,000 keys second:
+// D = 64, one 16-row block a tile, 14 / 2 heads: 388 tiles (3,100 tokens) 52 / 57
+// and 113 / 95, 450 (3,600) 69 / 70 and 130 / 110; 28 / 4 heads: 450 45 / 43 and
+// 101 / 80.  G = 1, 8 / 8 heads: 64 tiles (1,024) 21 / 30 and 57 / 64, 96 (1,536)
+// 32 / 30 and 64 / 44.  G = 2 to 4 keep more rows of a narrow item together: 8 / 2
+// heads, 388 tiles (6,200) 101 / 122 and 155 / 154.  D = 128, 14 / 2 heads: 80
+// tiles (640) 27 / 29 and 80 / 50, 96 (768) 31 / 33 and 84 / 54; two blocks a tile,
+// 32 / 8 heads: 64 tiles (256) 18 / 20 and 56 / 49, 72 (288) 23 / 21 and 76 / 45.
 static void wide_rule(MixedParams& p, int64_t D) {
   const int m = kWideColTiles / p.G;  // (G <= 8)
   const int64_t tiles = p.total_T * p.H_kv / (16 * m);
-  const int64_t enough = D <= 64 ? 128 * (p.G < 4 ? p.G : 4) : 96;
+  const int64_t enough = D > 64 ? (m > 1 ? 72 : 96) : m == 1 ? 448 : p.G == 1 ? 96 : 128 * (p.G < 4 ? p.G : 4);
   if (tiles < enough) return;
+  // a tile's partial region is addressed in 31 bits
+  if ((int64_t)16 * m * p.H_q * kWideMaxChunks * D * 4 > 0x7fffffff) return;
   p.wide_m = m;
   p.wide_wg = mixed_workgroups(p.H_kv, D <= 64 ? wide_waves_per_simd<64>() : wide_waves_per_simd<128>());
 }

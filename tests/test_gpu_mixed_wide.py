@@ -111,3 +111,31 @@ def test_wide_launch_past_max_seqlen(native_lib):
     assert err == 2  # CIE_ERRBIT_LEN
     want, _ = oracle_mixed(case)
     assert_attn_close(o[rows], want[rows], what="max_seqlen")
+
+
+SPLITS = {
+    # few rows over long prefixes: tiles of up to 8 chunks, the partial last tile among them
+    "d128-g7": (14, 2, 128, [9000, 6001, 0, 1500], [770, 30, 17, 1]),
+    "d128-g4": (32, 8, 128, [8015, 700, 3000], [290, 3, 1]),
+    "d64-g1": (8, 8, 64, [7000, 0, 2000], [1501, 70, 1]),
+}
+
+
+@pytest.mark.parametrize("name", SPLITS)
+def test_wide_launch_of_long_prefixes(native_lib, name):
+    """Tiles of several chunks, under the default partials budget, a third of it
+    (fewer, longer chunks) and none: every one matches the oracle."""
+    h_q, h_kv, d, prior, new = SPLITS[name]
+    case = inputs.make_case(prior, new, h_q=h_q, h_kv=h_kv, d=d, seed=95)
+    note(f"wide long prefixes {name}")
+    o, err = _run(case, h_q)
+    assert err == 0
+    want, written = oracle_mixed(case)
+    assert_attn_close(o[written], want[written], what=name)
+    c = case.to(DEV)
+    kp, vp = (t.to(DEV) for t in case.appended_pools())
+    full = native_lib.cie_mixed_partials_bytes(case.T, h_q, d)
+    for nbytes in (full // 3, 0):
+        o = mixed_gqa_attention(c.q, kp, vp, max(new), c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table,
+                                partials_bytes=nbytes)
+        assert_attn_close(o[0].float().cpu()[written], want[written], what=f"{name}, {nbytes} bytes")
