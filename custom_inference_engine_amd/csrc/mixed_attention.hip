@@ -576,7 +576,7 @@ __device__ __forceinline__ void run_wide(const MixedParams& p, const SeqInfo& s,
 #pragma unroll
   for (int c = 0; c < NCT; ++c) load_combo_q<D>(p, s, tp, g, ct0 + c, r16, grp, q[c], lim[c]);
   const bool live = ct0 < tp.n_ctiles;
-  stream_wide<D, NCT>(st, q, lim, kt0, kt1, tp.key_end, src, p.scale_log2, sm);
+  stream_wide<D, NCT>(st, q, lim, s.c + tp.row0 + 1, kt0, kt1, tp.key_end, src, p.scale_log2, sm);
   if (!live) return;
   const int lane = opaque((int)threadIdx.x) & (kWave - 1);
   r16 = lane & 15;

@@ -108,15 +108,45 @@ __device__ __forceinline__ void mask_wide(f32x4 (&s)[NCT][2], int key0, const in
     }
 }
 
+// P.V operands of the two key tiles at key0: rows of keys at or past lim
+// (wave-uniform) become zeros.  va[nt][e] is key key0 + 16 * (e / 4) + 4 * grp +
+// e % 4.
+template <int NT>
+__device__ __forceinline__ void zero_keys(f16x8 (&va)[NT], int key0, int lim, int grp) {
+  const int n = lim - key0 - 4 * grp;  // keys of the lane's first four that stay; 16 less: of the others
+  uint32_t keep[4];                    // a mask per pair of keys
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int m = n - (i & 1) * 2 - (i >> 1) * 16;
+    keep[i] = m <= 0 ? 0u : m == 1 ? 0xffffu : 0xffffffffu;
+  }
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    u32x4 w = __builtin_bit_cast(u32x4, va[nt]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] &= keep[i];
+    va[nt] = __builtin_bit_cast(f16x8, w);
+  }
+}
+
+template <bool B>
+struct Bool {
+  static constexpr bool value = B;
+};
+
 // Streams key tiles [t_begin, t_end) (t_begin even) of the workgroup's item
 // through every wave's NCT column tiles.  All waves call it with the same
-// bounds; a wave without columns attends with zero queries.  Columns attend keys below lim[c]; keys at or past key_end do not exist.
+// bounds; a wave without columns attends with zero queries.  Columns attend keys
+// below lim[c], which grows with the column from first_lim, the item's first
+// row's; keys at or past key_end do not exist.
 // sm: WideLds<D>::bytes, free for the workgroup to write when it is called;
 // it is free again when it returns.
 template <int D, int NCT>
 __device__ __forceinline__ void stream_wide(SoftmaxAcc<D, NCT>& st, const f16x8 (&q)[NCT][Geo<D>::KS],
-                                            const int (&lim)[NCT], int t_begin, int t_end, int key_end,
-                                            const PagedSrc& src, float scale_log2, f16* sm) {
+                                            const int (&lim)[NCT], int first_lim, int t_begin,
+                                            int t_end, int key_end, const PagedSrc& src,
+                                            float scale_log2, f16* sm) {
   constexpr int KS = Geo<D>::KS;
   constexpr int NT = Geo<D>::NT;
   constexpr int CH = D / 8;            // 16-byte chunks a row
@@ -136,12 +166,14 @@ __device__ __forceinline__ void stream_wide(SoftmaxAcc<D, NCT>& st, const f16x8 
   const int lane = opaque((int)threadIdx.x) & (kWave - 1);
   const int wave = uniform((int)threadIdx.x / kWave);
   const int r16 = lane & 15, grp = lane >> 4;
-  // the wave's smallest column limit: steps below it need no mask
-  int mask_from = kNoKey;
+  first_lim = uniform(first_lim);
+  // each column tile's largest limit (its last column's).  P is 0 past a column's
+  // limit, but 0 times an Inf or NaN in V is NaN, so V rows that no column of a
+  // tile attends are zeros for that tile: such a value reaches no row of an
+  // earlier 16-row block, as in a narrow launch (16 * G columns are whole tiles).
+  int v_end[NCT];
 #pragma unroll
-  for (int c = 0; c < NCT; ++c) mask_from = min(mask_from, lim[c]);
-  for (int off = 1; off < kWave; off <<= 1) mask_from = min(mask_from, __shfl_xor(mask_from, off, kWave));
-  mask_from = uniform(mask_from);
+  for (int c = 0; c < NCT; ++c) v_end[c] = __builtin_amdgcn_readlane(lim[c], 15);
 
   // staging: a lane moves the 16 bytes that its slot of the wave's RPW rows
   // holds (byte offsets inside a 16-key tile of the pool)
@@ -236,14 +268,13 @@ __device__ __forceinline__ void stream_wide(SoftmaxAcc<D, NCT>& st, const f16x8 
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) s[c][t] = mfma16x16x32(kf[t][ks], q[c][ks], s[c][t]);
       }
-    if (t_begin * 16 + 32 > mask_from) mask_wide<NCT>(s, t_begin * 16, lim, grp);
+    if (t_begin * 16 + 32 > first_lim) mask_wide<NCT>(s, t_begin * 16, lim, grp);
     update_max<D, NCT>(st, s, scale_log2);
     arguments(s);
   }
   // (no branch around a step's MFMAs: the compiler would keep two copies of
   // the accumulators)
-#pragma unroll 1
-  for (int step = 0; step < n_steps; ++step) {
+  auto do_step = [&](int step, auto masked) {
     // the next step's stage, if it is a new one, and the loads of the one after
     const int stg = (step + 1) / kSub;
     if ((step + 1) % kSub == 0 && stg < n_stages) {
@@ -286,16 +317,28 @@ __device__ __forceinline__ void stream_wide(SoftmaxAcc<D, NCT>& st, const f16x8 
       asm volatile("" : "+v"(pop[c]));
     }
     const int key0 = (t_begin + 2 * (step + 1)) * 16;
-    if (key0 + 32 > mask_from) mask_wide<NCT>(s, key0, lim, grp);
+    if constexpr (masked.value) mask_wide<NCT>(s, key0, lim, grp);
+    // (the later tile first: what is past its end is past the earlier one's)
 #pragma unroll
-    for (int c = 0; c < NCT; ++c) {
+    for (int c = NCT - 1; c >= 0; --c) {
+      if constexpr (masked.value) zero_keys<NT>(va, key0 - 32, v_end[c], grp);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) st.acc[c][nt] = mfma16x16x32(va[nt], pop[c], st.acc[c][nt]);
       add_row_sums(st.lpart[c], pop[c]);
     }
     if (step + 1 < n_steps) update_max<D, NCT>(st, s, scale_log2);
     arguments(s);
-  }
+  };
+  // A loop for the steps whose next one lies below every limit of the item (the
+  // same for all waves, which meet at a stage's barrier), and one for the others:
+  // tests for masking and for the V rows in every step cost 3-6 % at D = 64.
+  const int open = first_lim - 16 * t_begin - 32;
+  const int n_open = open < 32 ? 0 : min(n_steps, open / 32);
+  int step = 0;
+#pragma unroll 1
+  for (; step < n_open; ++step) do_step(step, Bool<false>());
+#pragma unroll 1
+  for (; step < n_steps; ++step) do_step(step, Bool<true>());
   __syncthreads();  // (the caller may write sm)
 }
 

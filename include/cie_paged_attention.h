@@ -316,7 +316,9 @@ int cie_kv_append_tokens_qkv_rope(void* q_out, void* k_pool, void* v_pool,
  * chunked-prefill and decode sequences.  Sequence b owns query rows
  * [cu_seqlens[b], cu_seqlens[b+1]); its row i sits at absolute position
  * kv_lens[b] + i and attends keys [0, kv_lens[b] + i] of slot slot_ids[b].
- * Rows outside every sequence are not written.
+ * Rows outside every sequence are not written.  An Inf or NaN in a key's V row
+ * reaches the rows that attend the key, and may reach the rows before them in
+ * the same 16 rows of the sequence (rows 16 * i .. 16 * i + 15); no others.
  * Replaces mixed_gqa_attention (attn/core.py:69-111), i.e. the Triton
  * mixed_gqa_attention_kernel (kernels/prefill_attention.py:10-198).
  *   q, o       : (total_T, H_q, D) dense fp16

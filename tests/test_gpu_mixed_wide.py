@@ -23,7 +23,7 @@ def _wide(case, h_q, h_kv, d):
     return tiles >= (96 if d == 128 else 128 * min(4, h_q // h_kv))
 
 
-def _run(case, h_q, max_seqlen=None, poison=False, rows=slice(None)):
+def _run(case, h_q, max_seqlen=None, poison=False, rows=slice(None), bad_v=()):
     c = case.to(DEV)
     kp, vp = c.k_pool.clone(), c.v_pool.clone()
     if poison:  # pool rows past each sequence's end hold NaN (as uninitialised memory may)
@@ -37,6 +37,10 @@ def _run(case, h_q, max_seqlen=None, poison=False, rows=slice(None)):
         vp.transpose(1, 2)[~used.to(DEV)] = float("nan")
     err = err_word()
     kv_append_tokens(kp, vp, c.k_new, c.v_new, c.pages, c.offsets, err=err)
+    for b, j in bad_v:  # V of new row j of sequence b
+        pos = int(case.kv_lens[b]) + j
+        row = vp[int(case.block_table[int(case.slot_ids[b]), pos // case.page_size]), :, pos % case.page_size]
+        row[:, 0::2], row[:, 1::2] = float("inf"), float("nan")
     ms = max_seqlen or int(case.new_lens.max())
     plan = mixed_plan(kp, c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table, ms, case.T, h_q, err=err)
     o = [mixed_gqa_attention(c.q, kp, vp, ms, c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table, err=err,
@@ -139,3 +143,36 @@ def test_wide_launch_of_long_prefixes(native_lib, name):
         o = mixed_gqa_attention(c.q, kp, vp, max(new), c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table,
                                 partials_bytes=nbytes)
         assert_attn_close(o[0].float().cpu()[written], want[written], what=f"{name}, {nbytes} bytes")
+
+
+MASKED = {  # h_q, h_kv, d, prior, new
+    "d64-g1": (8, 8, 64, [0, 37, 2000], [700, 500, 420]),
+    "d64-g2": (16, 8, 64, [0, 37, 2000], [700, 600, 800]),
+    "d64-g3": (24, 8, 64, [0, 37, 2000], [700, 600, 400]),
+    "d128-g1": (8, 8, 128, [0, 37, 3000], [900, 700, 500]),
+    "d128-g2": (16, 8, 128, [0, 37, 3000], [400, 300, 200]),
+    "d128-g4": (32, 8, 128, [0, 37, 3000], [200, 170, 130]),
+    "d128-g3": (24, 8, 128, [0, 37, 3000], [200, 170, 130]),
+    "d128-g7": (14, 2, 128, [0, 37, 3000], [500, 450, 300]),
+}
+
+
+@pytest.mark.parametrize("name", MASKED)
+def test_wide_launch_keeps_masked_values_out(native_lib, name):
+    """Inf and NaN in the V row of a new token reach no row of an earlier 16-row block of
+    its sequence: those rows are bit for bit what they are with finite values there."""
+    h_q, h_kv, d, prior, new = MASKED[name]
+    case = inputs.make_case(prior, new, h_q=h_q, h_kv=h_kv, d=d, seed=96)
+    m = 8 // (h_q // h_kv)
+    # the last block of a wide tile, the second block of one (its first row), the last row
+    first = [16 * m - 1 + 16 * m, 16 if m > 1 else 32, new[2] - 1]
+    note(f"wide masked {name}")
+    clean, err = _run(case, h_q)
+    assert err == 0
+    bad, err = _run(case, h_q, bad_v=list(enumerate(first)))
+    assert err == 0
+    for b, j in enumerate(first):
+        t0 = int(case.cu_seqlens[b])
+        before = slice(t0, t0 + j // 16 * 16)
+        assert torch.equal(bits(bad[before]), bits(clean[before])), (name, b)
+        assert not torch.isfinite(bad[t0 + j]).any(), (name, b)
