@@ -42,7 +42,8 @@
 namespace cie {
 
 // Build-time tuning (defaults are the shipped configuration):
-//   CIE_MIXED_WAVES        wavefronts per workgroup (D = 64)
+//   CIE_MIXED_WAVES        wavefronts per workgroup (D = 64; no launch is wide
+//                          unless it is the four that wide_tiles.h is laid out for)
 //   CIE_MIXED_CG           column tiles per work item (D = 64)
 //   CIE_MIXED_WAVE_PAIRS   32-key steps per wave before a tile's keys are
 //                          split over several workgroups
@@ -120,6 +121,13 @@ constexpr int64_t kMaxPartRows = (1 << 21) - 64;
 template <int D>
 constexpr int mixed_waves() {
   return D <= 64 ? CIE_MIXED_WAVES : 4;
+}
+// Whether this build has wide launches: their stages and column tiles are laid
+// out for kWideWaves waves (fewer would leave part of each stage unwritten, more
+// would write past it).
+template <int D>
+constexpr bool has_wide() {
+  return mixed_waves<D>() == kWideWaves;
 }
 template <int D>
 constexpr int col_group() {
@@ -1329,6 +1337,7 @@ template <int D, bool P32, bool kPlanned, bool kWide>
 __global__ __launch_bounds__(mixed_waves<D>() * kWave)
 __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixed_attention_kernel(
     MixedParams p) {
+  static_assert(!kWide || has_wide<D>(), "a wide item takes kWideWaves waves");
   static_assert(col_group<D>() <= 4 && 8 / col_group<D>() <= kMaxColGroups, "column groups");
   static_assert(mixed_lds_fits<D>(),
                 "static LDS + the plan tables of kMaxSeqs sequences exceed a workgroup's LDS");
@@ -1551,9 +1560,11 @@ static int launch_mixed_kernel(const MixedParams& p, hipStream_t stream) {
 
 template <int D, bool kPlanned>
 static int launch_mixed(const MixedParams& p, hipStream_t stream) {
-  if (p.wide_m > 0)
-    return p.pool_bytes != 0 ? launch_mixed_kernel<D, true, kPlanned, true>(p, stream)
-                             : launch_mixed_kernel<D, false, kPlanned, true>(p, stream);
+  if constexpr (has_wide<D>()) {
+    if (p.wide_m > 0)
+      return p.pool_bytes != 0 ? launch_mixed_kernel<D, true, kPlanned, true>(p, stream)
+                               : launch_mixed_kernel<D, false, kPlanned, true>(p, stream);
+  }
   return p.pool_bytes != 0 ? launch_mixed_kernel<D, true, kPlanned, false>(p, stream)
                            : launch_mixed_kernel<D, false, kPlanned, false>(p, stream);
 }
@@ -1658,6 +1669,7 @@ extern "C" int cie_mixed_trace_buffer(void* buf) {
 // tiles (640) 27 / 29 and 80 / 50, 96 (768) 31 / 33 and 84 / 54; two blocks a tile,
 // 32 / 8 heads: 64 tiles (256) 18 / 20 and 56 / 49, 72 (288) 23 / 21 and 76 / 45.
 static void wide_rule(MixedParams& p, int64_t D) {
+  if (!(D <= 64 ? has_wide<64>() : has_wide<128>())) return;
   const int m = kWideColTiles / p.G;  // (G <= 8)
   const int64_t tiles = p.total_T * p.H_kv / (16 * m);
   const int64_t enough = D > 64 ? (m > 1 ? 72 : 96) : m == 1 ? 448 : p.G == 1 ? 96 : 128 * (p.G < 4 ? p.G : 4);

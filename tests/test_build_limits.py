@@ -38,9 +38,25 @@ def test_mixed_build_past_the_lds_budget_does_not_compile(tmp_path):
     assert "exceed a workgroup's LDS" in res.stderr
 
 
+def _wide_kernels(stderr, d):
+    """Names of the D = d kernels that run wide items (the last template argument)."""
+    return set(re.findall(rf"mixed_attention_kernelILi{d}ELb[01]ELb[01]ELb1EE", stderr))
+
+
+@pytest.mark.parametrize("waves", [2, 8])
+def test_mixed_build_of_other_wave_counts_has_no_wide_launch(tmp_path, waves):
+    """Wide items are laid out for four waves: with two, half of each K/V stage would stay
+    unwritten, with eight the stages would be written past their end."""
+    res = _compile(tmp_path, f"CIE_MIXED_WAVES={waves}", "CIE_MIXED_CG=2")
+    assert res.returncode == 0, res.stderr[-3000:]
+    assert not _wide_kernels(res.stderr, 64)
+    assert _wide_kernels(res.stderr, 128)  # always four waves
+
+
 def test_shipped_mixed_build_plans_its_largest_batch_within_lds(tmp_path):
     res = _compile(tmp_path)
     assert res.returncode == 0, res.stderr[-3000:]
+    assert len(_wide_kernels(res.stderr, 64)) == len(_wide_kernels(res.stderr, 128)) == 4
     sizes = [int(m) for m in re.findall(r"mixed_attention_kernel\w*.*?\n.*?LDS Size \[bytes/block\]: (\d+)",
                                         res.stderr, flags=re.S)]
     if not sizes:  # remarks printed in another order: take every LDS size line of the file
