@@ -217,6 +217,9 @@ template <int D, int NTHREADS, bool kMany>
 __device__ __forceinline__ void merge_splits(const DecodeParams& p, const PartRows& prow, int b,
                                              int g, int n_splits, int n_states, int tid,
                                              f32x4* sm);
+// f32x4 of LDS that the merge of many splits takes: a float a (head, split) and a
+// sum a thread (merge_many)
+constexpr int merge_words(int n_threads) { return 16 * kMaxSplits / 4 + n_threads; }
 
 // Profiling builds only (-DCIE_DECODE_TRACE): phase boundaries
 // (s_memrealtime) are stamped into LDS — LDS writes do not count in vmcnt, so
@@ -279,8 +282,13 @@ void decode_kernel(const int64_t* __restrict__ a_slot_ids, const int32_t* __rest
   constexpr int NT = Geo<D>::NT;
   __shared__ float sm_m[WAVES][16];
   __shared__ float sm_l[WAVES][16];
-  // rows padded to keep 16-byte alignment for the vector reads of the fold
-  __shared__ f32x4 sm_acc[WAVES][16][D / 4 + 1];
+  // rows padded to keep 16-byte alignment for the vector reads of the fold; the
+  // merge of many splits uses the array as its scratch (a build of one wave at
+  // D = 64 needs more than the fold does)
+  constexpr int kAccRow = 16 * (D / 4 + 1);
+  constexpr int kMergeRows = kMany ? (merge_words(WAVES * kWave) + kAccRow - 1) / kAccRow : 0;
+  constexpr int kAccRows = WAVES > kMergeRows ? WAVES : kMergeRows;
+  __shared__ f32x4 sm_acc[kAccRows][16][D / 4 + 1];
   __shared__ int sm_last;
 #ifdef CIE_DECODE_TRACE
   __shared__ uint64_t sm_trace[kTraceSlots];
@@ -732,7 +740,8 @@ __device__ __forceinline__ void merge_few(const DecodeParams& p, const PartRows&
 // together with the m and l loads.  Those take one split a lane (kMaxSplits =
 // the wave): a wave reduces a head's max and sum across lanes, and the splits'
 // weights 2^(m - M) / l go to LDS, so no thread repeats them.
-// sm: 16 * kMaxSplits floats of weights, then NTHREADS f32x4 of partial sums.
+// sm (merge_words): 16 * kMaxSplits floats of weights, then NTHREADS f32x4 of
+// partial sums.
 constexpr int kMergeLoads = 16;
 
 template <int D, int NTHREADS>

@@ -22,12 +22,13 @@ from custom_inference_engine_amd import _build
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
 SRC = os.path.join(_build.CSRC, "mixed_attention.hip")
+DECODE = os.path.join(_build.CSRC, "paged_decode.hip")
 
 
-def _compile(tmp_path, *defines):
+def _compile(tmp_path, *defines, src=SRC):
     flags = [f for f in _build.HIPCC_FLAGS if f != "-fPIC"]
     cmd = [HIPCC, *flags, *(f"-D{d}" for d in defines), "-I", _build.INCLUDE, "-I", _build.CSRC,
-           "--offload-device-only", "-c", SRC, "-o", str(tmp_path / "mixed.o"),
+           "--offload-device-only", "-c", src, "-o", str(tmp_path / "kernels.o"),
            "-Rpass-analysis=kernel-resource-usage"]
     return subprocess.run(cmd, capture_output=True, text=True)
 
@@ -66,3 +67,17 @@ def test_shipped_mixed_build_plans_its_largest_batch_within_lds(tmp_path):
     plan = k_max_seqs * 8 + (4 * k_max_seqs + k_max_seqs + 1) * 4
     for static in sizes:
         assert static + plan <= 160 * 1024, (static, plan)
+
+
+@pytest.mark.parametrize("waves", [1, 4])
+def test_decode_merge_of_many_splits_fits_its_lds(tmp_path, waves):
+    """The merge keeps a float for each of 16 heads x 64 splits and 16 bytes a thread in the
+    fold's LDS, which a one-wave build's fold alone does not fill."""
+    res = _compile(tmp_path, f"CIE_DECODE_WAVES={waves}", src=DECODE)
+    assert res.returncode == 0, res.stderr[-3000:]
+    many = re.findall(r"decode_kernelILi(\d+)ELi(\d+)ELb[01]ELb[01]ELb[01]ELb1EE.*?LDS Size \[bytes/block\]: (\d+)",
+                      res.stderr, flags=re.S)
+    assert any(int(w) == waves for _, w, _ in many)
+    for d, w, lds in many:
+        rest = 2 * int(w) * 16 * 4 + 4  # the waves' maxima and sums, the arrival flag
+        assert int(lds) - rest >= 16 * 64 * 4 + int(w) * 64 * 16, (d, w, lds)
