@@ -703,6 +703,9 @@ constexpr int kMaxSeqs = 1024;  // sequences a launch can plan (LDS plan tables)
 // rounds in LDS.
 constexpr int kPlanHeader = 8;
 constexpr int kDescRounds = 16;
+// An unplanned wide launch makes the descriptors of so many of a workgroup's
+// rounds at a time, a round a lane (own_plan in the kernel).
+constexpr int kOwnRounds = kWave;
 constexpr int kRankSeqs = 64;   // batches up to this size deal their items heaviest first
 static_assert(kRankSeqs == kWave, "a batch small enough to rank is planned by one wave");
 
@@ -1090,8 +1093,7 @@ struct MixedLds {
 // line of defence for devices with less.)
 template <int D>
 constexpr bool mixed_lds_fits() {
-  return MixedLds<D, false>::bytes + mixed_plan_lds(kMaxSeqs) <= kLdsPerWorkgroup &&
-         MixedLds<D, true>::bytes + mixed_plan_lds(kMaxSeqs) <= kLdsPerWorkgroup;
+  return MixedLds<D, false>::bytes + mixed_plan_lds(kMaxSeqs) <= kLdsPerWorkgroup;
 }
 
 // The batch's plan tables in LDS (sm_plan, mixed_plan_lds(B) bytes), all by
@@ -1138,6 +1140,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
   constexpr int NTH = W * kWave;
   constexpr int CG = col_group<D>();
   const int B = p.B;
+  const int tid = opaque((int)threadIdx.x);  // (a kernel that plans in its item loop would keep its terms)
   int2* const sm_tp = t.tp;
   int* const sm_slot = t.slot;
   int* const sm_rows = t.rows;
@@ -1149,7 +1152,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
     // A batch of up to 64 sequences: every wave plans it alone, a lane per
     // sequence, and writes the same tables (identical values from every
     // wave), reading back only what it wrote itself — no barrier.
-    const int lane = threadIdx.x & (kWave - 1);
+    const int lane = tid & (kWave - 1);
     int n = 0, key = -1, prows = 0;
     SeqInfo s{0, 0, 0, 0, 0, 0, 0};  // pbase 0: counted as split
     if (lane < B) s = seq_info(p, lane);
@@ -1160,7 +1163,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
     }
     s.q = wide_q;
     if (lane < B) {
-      if (blockIdx.x == 0 && threadIdx.x < kWave && ((s.L + 15) >> 4) > p.n_qtiles)
+      if (blockIdx.x == 0 && tid < kWave && ((s.L + 15) >> 4) > p.n_qtiles)
         set_err(p.err, CIE_ERRBIT_LEN);  // rows past max_seqlen are not computed
       int weight = 0;
       if (s.L > 0)
@@ -1241,14 +1244,14 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
     wide_q = 0;
     if (p.wide_m > 0) {
       WideWork w{0.f, 0.f};
-      for (int b = threadIdx.x; b < B; b += NTH) {
+      for (int b = tid; b < B; b += NTH) {
         const WideWork x = wide_work(p, seq_info(p, b));
         w.tiles += x.tiles;
         w.ktiles += x.ktiles;
       }
       w = {wave_sum(w.tiles), wave_sum(w.ktiles)};
       float2* const sm = reinterpret_cast<float2*>(sm_scan);
-      if ((threadIdx.x & (kWave - 1)) == 0) sm[threadIdx.x / kWave] = float2{w.tiles, w.ktiles};
+      if ((tid & (kWave - 1)) == 0) sm[tid / kWave] = float2{w.tiles, w.ktiles};
       __syncthreads();
       w = {0.f, 0.f};
 #pragma unroll
@@ -1259,7 +1262,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
       wide_q = uniform(wide_share<D>(p, w));
       __syncthreads();
     }
-    for (int b = threadIdx.x; b < B; b += NTH) {
+    for (int b = tid; b < B; b += NTH) {
       SeqInfo s = seq_info(p, b);  // pbase 0: counted as split
       s.q = wide_q;
       sm_tp[b].x = (int)s.t0;
@@ -1278,7 +1281,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
     __syncthreads();
     int ptot = 0;
     for (int q0 = 0; q0 < B; q0 += NTH) {
-      const int q = q0 + threadIdx.x;
+      const int q = q0 + tid;
       const int2 c = q < B ? int2{sm_prefix[q + 1], sm_tp[q].y} : int2{0, 0};
       const int span = min(NTH, B - q0);
       const int2 inc = block_scan2<NTH>(c, sm_scan, span);
@@ -1295,7 +1298,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
       // The batch's split tiles need more partial rows than the buffer
       // holds: a sequence whose rows end past it runs unsplit; its item
       // count is taken again and the item prefix scanned again.
-      for (int b = threadIdx.x; b < B; b += NTH) {
+      for (int b = tid; b < B; b += NTH) {
         SeqInfo s;
         s.t0 = sm_tp[b].x;
         s.slot = sm_slot[b];
@@ -1317,7 +1320,7 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
       __syncthreads();
       base = 0;
       for (int q0 = 0; q0 < B; q0 += NTH) {
-        const int q = q0 + threadIdx.x;
+        const int q = q0 + tid;
         const int c = q < B ? sm_prefix[q + 1] : 0;
         const int span = min(NTH, B - q0);
         const int2 inc = block_scan2<NTH>(int2{c, 0}, sm_scan, span);
@@ -1327,10 +1330,38 @@ __device__ __forceinline__ int plan_batch(const MixedParams& p, const PlanTables
         __syncthreads();
       }
     }
-    if (threadIdx.x == 0) sm_prefix[0] = 0;
+    if (tid == 0) sm_prefix[0] = 0;
     __syncthreads();
   }
   return uniform(base);
+}
+
+// Item i's descriptor, from the batch's plan (each thread its own item).
+template <int D>
+__device__ __forceinline__ void item_desc(const MixedParams& p, const PlanTables& t, int wide_q, int i,
+                                          int4& d0, int4& d1) {
+  constexpr int W = mixed_waves<D>();
+  constexpr int CG = col_group<D>();
+  // the last position whose prefix is at or below i (prefix[0] = 0)
+  int lo = 0, hi = p.B - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (t.prefix[mid] <= i) lo = mid;
+    else hi = mid - 1;
+  }
+  const int2 tb = t.tp[lo];
+  SeqInfo s;
+  s.t0 = tb.x;
+  s.slot = t.slot[lo];
+  s.L = t.rows[lo];
+  s.c = t.prior[lo];
+  s.pbase = tb.y;
+  s.m = seq_blocks(p, s.L);
+  s.q = wide_q;
+  int qt, jt;
+  seq_locate<CG, W>(p, s, seq_tiles<CG, W>(p, s), i - t.prefix[lo], qt, jt);
+  d0 = int4{t.order[lo], qt, jt, (int)s.t0};
+  d1 = int4{(int)s.slot, s.L, s.c, s.pbase};
 }
 
 template <int D, bool P32, bool kPlanned, bool kWide>
@@ -1356,9 +1387,18 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
   // Unplanned launches: the plan tables, in LDS sized by the launch to the
   // batch (mixed_plan_lds).  Planned launches: the descriptors of this
   // workgroup's first kDescRounds items.
+  // Unplanned wide launches: the tables lie where the items' stages will, and
+  // the descriptors of the workgroup's next kOwnRounds items are made from them
+  // before the first of these starts.  (Tables of their own cost a CU one of its
+  // workgroups from 91 sequences on, D = 128: 512, and the items dealt to it ran
+  // after the others'.  us a call in 16-row tiles / wide with such tables / so:
+  // 14 / 2 heads, D = 64, 96 chunks of 39 rows over 2,000 keys 88 / 100 / 89, 250 of
+  // 33 on nothing 89 / 51 / 37; 32 / 8 heads, D = 128, 530 of 3 100 / 113 / 68.)
+  constexpr bool kOwnPlan = kWide && !kPlanned;
+  static_assert(!kOwnPlan || Lds::words * 16 >= mixed_plan_lds(kMaxSeqs), "plan tables fit the stages");
   extern __shared__ __attribute__((aligned(16))) char sm_plan[];
-  __shared__ __attribute__((aligned(16))) int4 sm_desc[kPlanned ? 2 * kDescRounds : 1];
-  const PlanTables tables(sm_plan, p.B);
+  __shared__ __attribute__((aligned(16))) int4 sm_desc[kPlanned ? 2 * kDescRounds : kOwnPlan ? 2 * kOwnRounds : 1];
+  const PlanTables tables(kOwnPlan ? reinterpret_cast<char*>(sm_facc) : sm_plan, p.B);
 
   // (known to the compiler: no item of a narrow launch is wide.  A division by
   // the wide chunk length, taken per item ahead of the test, cost 2 %)
@@ -1383,7 +1423,19 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
     const int r = q * kPerCu + layer;
     return r * n_cu_r + ((r & 1) ? n_cu_r - 1 - cu_r : cu_r);
   };
-  int n_items, wide_q;
+  int n_items = 0, wide_q = 0;
+  // this workgroup's descriptors of rounds [q0, q0 + kOwnRounds)
+  auto own_plan = [&](int q0) {
+    __syncthreads();  // the item before may still be in the stages
+    n_items = plan_batch<D>(p, tables, sm_scan, wide_q);
+    __syncthreads();
+    const int tid = threadIdx.x;
+    if (tid < kOwnRounds) {
+      const int it = item_of(q0 + tid);
+      if (it < n_items) item_desc<D>(p, tables, wide_q, it, sm_desc[2 * tid], sm_desc[2 * tid + 1]);
+    }
+    __syncthreads();
+  };
   if constexpr (kPlanned) {
     // The step's plan: a header, then one 8-word descriptor per item.  The
     // header and the descriptors of this workgroup's first kDescRounds
@@ -1408,7 +1460,7 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
       if (blockIdx.x == 0 && threadIdx.x == 0) set_err(p.err, CIE_ERRBIT_PLAN);
       return;
     }
-  } else {
+  } else if constexpr (!kOwnPlan) {
     n_items = plan_batch<D>(p, tables, sm_scan, wide_q);
   }
   MIXED_TRACE(0, 6, __builtin_amdgcn_s_memrealtime());  // planning done
@@ -1419,14 +1471,21 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
   // workgroups that took the heaviest items of round 0 take the lightest of
   // round 1.
   for (int q = 0; slot_r < n_slots_r; ++q) {
+    if constexpr (kOwnPlan) {
+      if (q % kOwnRounds == 0) own_plan(q);
+    }
     const int item = item_of(q);
     if (item >= n_items) break;
     MIXED_TRACE(item, 0, __builtin_amdgcn_s_memrealtime());
     int b, qt, jt;
     SeqInfo s;
-    if constexpr (kPlanned) {
+    if constexpr (kPlanned || kOwnPlan) {
       int4 d0, d1;
-      if (q < kDescRounds) {
+      if constexpr (kOwnPlan) {
+        const int r = q % kOwnRounds;
+        d0 = sm_desc[2 * r];
+        d1 = sm_desc[2 * r + 1];
+      } else if (q < kDescRounds) {
         d0 = sm_desc[2 * q];
         d1 = sm_desc[2 * q + 1];
       } else {
@@ -1467,7 +1526,6 @@ template <int D>
 __global__ __launch_bounds__(mixed_waves<D>() * kWave) void mixed_plan_kernel(MixedParams p) {
   constexpr int W = mixed_waves<D>();
   constexpr int NTH = W * kWave;
-  constexpr int CG = col_group<D>();
   typedef MixedLds<D, false> Lds;
   __shared__ __attribute__((aligned(16))) int2 sm_scan[Lds::scan];
   extern __shared__ __attribute__((aligned(16))) char sm_plan[];
@@ -1486,27 +1544,8 @@ __global__ __launch_bounds__(mixed_waves<D>() * kWave) void mixed_plan_kernel(Mi
   }
   if (!fits) return;
   for (int i = threadIdx.x; i < n_items; i += NTH) {
-    // the last position whose prefix is at or below i (prefix[0] = 0)
-    int lo = 0, hi = p.B - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (t.prefix[mid] <= i) lo = mid;
-      else hi = mid - 1;
-    }
-    const int2 tb = t.tp[lo];
-    SeqInfo s;
-    s.t0 = tb.x;
-    s.slot = t.slot[lo];
-    s.L = t.rows[lo];
-    s.c = t.prior[lo];
-    s.pbase = tb.y;
-    s.m = seq_blocks(p, s.L);
-    s.q = wide_q;
-    int qt, jt;
-    seq_locate<CG, W>(p, s, seq_tiles<CG, W>(p, s), i - t.prefix[lo], qt, jt);
-    int32_t* const d = out + kPlanHeader + (int64_t)i * 8;
-    *reinterpret_cast<int4*>(d) = int4{t.order[lo], qt, jt, (int)s.t0};
-    *reinterpret_cast<int4*>(d + 4) = int4{(int)s.slot, s.L, s.c, s.pbase};
+    int4* const d = reinterpret_cast<int4*>(out + kPlanHeader + (int64_t)i * 8);
+    item_desc<D>(p, t, wide_q, i, d[0], d[1]);
   }
 }
 
@@ -1551,7 +1590,8 @@ static int launch_mixed_kernel(const MixedParams& p, hipStream_t stream) {
   // a batch whose plan tables would take the workgroup past the device's
   // LDS is refused here (the dispatch itself would be rejected); a planned
   // launch reads its plan instead of building the tables
-  const size_t dyn = kPlanned ? 0 : mixed_plan_lds(p.B);
+  // (a wide one's lie in its stages)
+  const size_t dyn = kPlanned || kWide ? 0 : mixed_plan_lds(p.B);
   if (lds + (int64_t)dyn > device_lds_limit()) return CIE_EUNSUPPORTED;
   hipLaunchKernelGGL((mixed_attention_kernel<D, P32, kPlanned, kWide>), grid,
                      dim3(mixed_waves<D>() * kWave), dyn, stream, p);

@@ -65,6 +65,13 @@ def test_shipped_mixed_build_plans_its_largest_batch_within_lds(tmp_path):
     assert sizes
     k_max_seqs = 1024  # kMaxSeqs: the ABI's batch limit for cie_mixed_attention
     plan = k_max_seqs * 8 + (4 * k_max_seqs + k_max_seqs + 1) * 4
+    # three wide workgroups a CU at D = 64, two at D = 128 (LDS goes in 1,280 bytes; the
+    # plan tables of a wide launch lie in its stages)
+    wide = re.findall(r"mixed_attention_kernelILi(\d+)ELb[01]ELb[01]ELb1EE.*?LDS Size \[bytes/block\]: (\d+)",
+                      res.stderr, flags=re.S)
+    assert len(wide) == 8
+    for d, static in wide:
+        assert 160 * 1024 // (-(-int(static) // 1280) * 1280) >= (3 if d == "64" else 2), (d, static)
     for static in sizes:
         assert static + plan <= 160 * 1024, (static, plan)
 

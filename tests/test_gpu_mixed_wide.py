@@ -176,3 +176,23 @@ def test_wide_launch_keeps_masked_values_out(native_lib, name):
         before = slice(t0, t0 + j // 16 * 16)
         assert torch.equal(bits(bad[before]), bits(clean[before])), (name, b)
         assert not torch.isfinite(bad[t0 + j]).any(), (name, b)
+
+
+OWN_PLANS = {  # heads (G = 1), d, workgroups a kv head on 256 CUs, prior, new
+    "d64": (256, 64, 3, [i % 9 for i in range(200)], [200 if i == 70 else 1 + i % 3 for i in range(200)]),
+    "d128": (256, 128, 2, [i % 9 for i in range(135)], [200 if i == 70 else 1 + i % 3 for i in range(135)]),
+}
+
+
+@pytest.mark.parametrize("name", OWN_PLANS)
+def test_wide_launch_plans_a_workgroups_rounds_in_parts(native_lib, name):
+    """Unplanned wide launches make the descriptors of 64 rounds of a workgroup at a time:
+    with few workgroups a kv head, a large batch has more rounds than that."""
+    h, d, slots, prior, new = OWN_PLANS[name]
+    case = inputs.make_case(prior, new, h_q=h, h_kv=h, d=d, seed=97)
+    assert len(new) > 64 * slots  # an item at least for each sequence
+    note(f"wide own plan {name}")
+    o, err = _run(case, h)
+    assert err == 0
+    want, written = oracle_mixed(case)
+    assert_attn_close(o[written], want[written], what=name)
