@@ -178,6 +178,7 @@ struct MixedParams {
   uint32_t g_magic, tpp_magic;  // div_magic(G), div_magic(page_size / 16)
   uint32_t pool_bytes;          // bytes of each pool if under 4 GiB, else 0
   int32_t wide_m;  // 16-row blocks of a wide query tile (wide_rule); 0: the launch has none
+  int32_t wide_ct;  // column tiles a wide item holds at most (a column group)
   int32_t wide_wg;  // workgroups of a wide launch
   float scale_log2;
   int32_t* err;
@@ -276,8 +277,8 @@ __device__ __forceinline__ TilePlan tile_plan(const MixedParams& p, int qt, cons
   t.rows = min(block, (wide ? seq_rows(p, s.L) : s.L) - t.row0);
   t.n_combos = t.rows * p.G;
   t.n_ctiles = (t.n_combos + 15) >> 4;
-  t.cg = wide ? kWideColTiles : seq_cg<CG>(s);
-  t.n_groups = wide ? 1 : n_col_groups<CG>(t.n_ctiles, t.cg);
+  t.cg = wide ? p.wide_ct : seq_cg<CG>(s);
+  t.n_groups = wide ? 1 + (t.n_ctiles > t.cg) : n_col_groups<CG>(t.n_ctiles, t.cg);
   t.key_end = s.c + t.row0 + t.rows;
   t.n_ktiles = (t.key_end + 15) >> 4;
   t.n_pairs = (t.n_ktiles + 1) >> 1;
@@ -753,7 +754,7 @@ __device__ __forceinline__ SeqTiles seq_tiles(const MixedParams& p, const SeqInf
     const int rows = seq_rows(p, s.L);
     t.n_full = rows / (16 * s.m);
     t.n_tiles = t.n_full + (t.n_full * 16 * s.m < rows ? 1 : 0);
-    t.ng_full = 1;
+    t.ng_full = 1 + (s.m * p.G > p.wide_ct);
     t.full_narrow = false;
   } else {
     t.n_tiles = min((s.L + 15) >> 4, p.n_qtiles);
@@ -1000,11 +1001,11 @@ __device__ __forceinline__ void process_item(const MixedParams& p, const SeqInfo
   if (wide) {
     f16* const sm = reinterpret_cast<f16*>(sm_facc);
     __syncthreads();  // the previous item's fold may still be reading its slots
-    const int per = (tp.n_ctiles + kWideWaves - 1) / kWideWaves;  // column tiles a wave
+    const int per = (n + kWideWaves - 1) / kWideWaves;  // column tiles a wave
     if (per <= 1)
-      run_wide<D, 1>(p, s, tp, g, wave, chunk, kt0, kt1, src, r16, grp, sm);
+      run_wide<D, 1>(p, s, tp, g, ct0 + wave, chunk, kt0, kt1, src, r16, grp, sm);
     else
-      run_wide<D, 2>(p, s, tp, g, 2 * wave, chunk, kt0, kt1, src, r16, grp, sm);
+      run_wide<D, 2>(p, s, tp, g, ct0 + 2 * wave, chunk, kt0, kt1, src, r16, grp, sm);
   } else if constexpr (kWide) {  // one column tile (seq_blocks)
     run_group<D, P32, 1>(p, s, tp, g, ct0, chunk, w0, w1, src, wave, r16, grp, sm_facc, sm_fml, sm_q,
                          item);
@@ -1042,7 +1043,7 @@ __device__ __forceinline__ void process_item(const MixedParams& p, const SeqInfo
     MIXED_TRACE(item, 4, __builtin_amdgcn_s_memrealtime());
     if (wide) {  // in blocks of column tiles that keep four units a thread
       constexpr int kBlock = D <= 64 ? 4 : 2;
-      for (int c = 0; c < tp.n_ctiles; c += kBlock)
+      for (int c = ct0; c < ct0 + n; c += kBlock)
         merge_group<D, kBlock>(p, s, tp, g, c, min(16 * kBlock, tp.n_combos - 16 * c));
     } else {
       merge_group<D, kWide ? 1 : col_group<D>()>(p, s, tp, g, ct0,
@@ -1364,6 +1365,11 @@ __device__ __forceinline__ void item_desc(const MixedParams& p, const PlanTables
   d1 = int4{(int)s.slot, s.L, s.c, s.pbase};
 }
 
+// How wide a plan's items are (0: not): a planned launch must agree.
+__device__ __forceinline__ int plan_wide_word(const MixedParams& p) {
+  return p.wide_m > 0 ? p.wide_ct * 16 + p.wide_m : 0;
+}
+
 template <int D, bool P32, bool kPlanned, bool kWide>
 __global__ __launch_bounds__(mixed_waves<D>() * kWave)
 __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixed_attention_kernel(
@@ -1455,7 +1461,7 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
     wide_q = max(1, uniform(h1.w));
     // a plan made for another batch shape, budget or partial layout
     if (uniform(h0.y) != (int)p.part_cap || uniform(h0.z) != p.B || uniform(h0.w) != p.n_qtiles ||
-        uniform(h1.x) != p.H_q || uniform(h1.y) != p.H_kv || uniform(h1.z) != p.wide_m ||
+        uniform(h1.x) != p.H_q || uniform(h1.y) != p.H_kv || uniform(h1.z) != plan_wide_word(p) ||
         n_items > p.plan_cap) {
       if (blockIdx.x == 0 && threadIdx.x == 0) set_err(p.err, CIE_ERRBIT_PLAN);
       return;
@@ -1520,7 +1526,7 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
 // A step's plan for its planned mixed launches (cie_mixed_plan): one
 // workgroup plans the batch as every workgroup of an unplanned launch does,
 // then writes the header {items, partial budget (rows), B, query tiles,
-// H_q, H_kv, wide_m, wide_q} and, per item in dealing order, its descriptor
+// H_q, H_kv, plan_wide_word, wide_q} and, per item in dealing order, its descriptor
 // {b, query tile, index in tile, t0, slot, rows, prior, partial base}.
 template <int D>
 __global__ __launch_bounds__(mixed_waves<D>() * kWave) void mixed_plan_kernel(MixedParams p) {
@@ -1540,7 +1546,7 @@ __global__ __launch_bounds__(mixed_waves<D>() * kWave) void mixed_plan_kernel(Mi
     // sequences can exceed it) gets an empty plan and CIE_ERRBIT_PLAN
     if (!fits) set_err(p.err, CIE_ERRBIT_PLAN);
     *reinterpret_cast<int4*>(out) = int4{fits ? n_items : 0, (int)p.part_cap, p.B, p.n_qtiles};
-    *reinterpret_cast<int4*>(out + 4) = int4{p.H_q, p.H_kv, p.wide_m, wide_q};
+    *reinterpret_cast<int4*>(out + 4) = int4{p.H_q, p.H_kv, plan_wide_word(p), wide_q};
   }
   if (!fits) return;
   for (int i = threadIdx.x; i < n_items; i += NTH) {
@@ -1694,29 +1700,42 @@ extern "C" int cie_mixed_trace_buffer(void* buf) {
 }
 #endif
 
-// Whether a launch is wide (see wide_tiles.h), from the number of wide tiles
-// that total_T rows make if they are all prefill: enough of them must fill the
-// chip, as a wide tile runs a longer serial loop than a narrow one.  The line
-// lies lower where narrow items share their keys among fewer columns: a narrow
-// item holds 4 column tiles at D = 64 (G at most, for G < 4), 1 at D = 128.
-// Measured, us a call with its append, narrow / wide, below a line and past it,
-// one prompt of n tokens on nothing first, the same over 2,000 keys second:
-// D = 64, one 16-row block a tile, 14 / 2 heads: 388 tiles (3,100 tokens) 52 / 57
-// and 113 / 95, 450 (3,600) 69 / 70 and 130 / 110; 28 / 4 heads: 450 45 / 43 and
-// 101 / 80.  G = 1, 8 / 8 heads: 64 tiles (1,024) 21 / 30 and 57 / 64, 96 (1,536)
-// 32 / 30 and 64 / 44.  G = 2 to 4 keep more rows of a narrow item together: 8 / 2
-// heads, 388 tiles (6,200) 101 / 122 and 155 / 154.  D = 128, 14 / 2 heads: 80
-// tiles (640) 27 / 29 and 80 / 50, 96 (768) 31 / 33 and 84 / 54; two blocks a tile,
-// 32 / 8 heads: 64 tiles (256) 18 / 20 and 56 / 49, 72 (288) 23 / 21 and 76 / 45.
-static void wide_rule(MixedParams& p, int64_t D) {
+// Whether a launch is wide (see wide_tiles.h), from its columns (row, q head) if
+// every row is prefill: a wide item runs a longer serial loop than a narrow one,
+// so a launch is wide where narrow items need one more round of the CUs than the
+// wide ones' time is worth.  A narrow item holds 64 columns at D = 64 (16 * G for
+// G < 4), 16 at D = 128, so a round of 256 CUs is 16,384 (4,096 * G) and 4,096
+// columns; the lines are whole rounds of them.
+// Measured, us a call with its append, one prompt on nothing, narrow / wide on
+// either side of a line; in brackets the same rows over 2,000 keys.
+// D = 64: G = 1, 8 / 8 heads, 12,288 columns: 1,345 rows 30 / 30, 1,560 35 / 30
+// [75 / 44].  G = 2, 16 / 8, 32,768: 1,901 44 / 37, 2,205 55 / 41 [107 / 63].  G > 2,
+// 49,152: 24 / 8 1,978 49 / 50, 2,294 62 / 60 [147 / 105]; 20 / 4 2,046 50 / 51, 2,753
+// 76 / 69; 14 / 2 3,391 66 / 68, 3,933 88 / 84 [154 / 122]; 12 / 4 2,940 49 / 56.
+// D = 128, 8,192: 32 / 8 251 19 / 20, 276 23 / 21 [75 / 44].  From there to 12,288 the
+// fewer heads that make a prompt's columns, the longer its serial loops: 20 / 4 487
+// rows 26 / 26, 16 / 8 608 28 / 29, 14 / 2 765 31 / 33, 8 / 8 1,217 35 / 40.  Such a launch
+// (less than kWideLongRatio columns for each row of its longest prompt) takes
+// items of half the columns, one column tile a wave: 16 / 8 608 25, 14 / 2 765 28
+// [83 / 63], 8 / 8 1,217 32.  Half as many columns read the keys twice as often:
+// 24 / 8, 385 rows over 2,000 keys 49 with all 8 column tiles, 60 so.
+// Batches of short chunks and of decode rows are faster wide from the same lines
+// (8 / 8 heads, D = 64, 95 chunks of 17 rows over 2,000 keys 158 / 91; 32 / 8, D =
+// 128, 71 of 5 160 / 156; 400 decode rows of 100 keys 78 / 63).
+constexpr int64_t kWideLongRatio = 20;
+static void wide_rule(MixedParams& p, int64_t max_seqlen, int64_t D) {
   if (!(D <= 64 ? has_wide<64>() : has_wide<128>())) return;
-  const int m = kWideColTiles / p.G;  // (G <= 8)
-  const int64_t tiles = p.total_T * p.H_kv / (16 * m);
-  const int64_t enough = D > 64 ? (m > 1 ? 72 : 96) : m == 1 ? 448 : p.G == 1 ? 96 : 128 * (p.G < 4 ? p.G : 4);
-  if (tiles < enough) return;
+  const int64_t columns = p.total_T * p.H_q;
+  const int64_t line = D > 64 ? 8192 : p.G == 1 ? 12288 : p.G == 2 ? 32768 : 49152;
+  if (columns <= line) return;
+  const int64_t longest = max_seqlen < p.total_T ? max_seqlen : p.total_T;
+  const int ct = D > 64 && columns <= 12288 && columns < kWideLongRatio * longest ? kWideColTiles / 2
+                                                                                  : kWideColTiles;
+  const int m = ct > p.G ? ct / p.G : 1;  // (G <= 8)
   // a tile's partial region is addressed in 31 bits
   if ((int64_t)16 * m * p.H_q * kWideMaxChunks * D * 4 > 0x7fffffff) return;
   p.wide_m = m;
+  p.wide_ct = ct;
   p.wide_wg = mixed_workgroups(p.H_kv, D <= 64 ? wide_waves_per_simd<64>() : wide_waves_per_simd<128>());
 }
 
@@ -1756,7 +1775,7 @@ static int mixed_shape(MixedParams& p, int64_t B, int64_t total_T, int64_t max_s
   // The buffer sets the budget of partial rows: sequences whose split tiles
   // do not fit run unsplit (the plan's pbase).
   p.part_cap = mixed_partial_rows(partials_bytes, D);
-  wide_rule(p, D);
+  wide_rule(p, max_seqlen, D);
   return CIE_OK;
 }
 

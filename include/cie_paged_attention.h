@@ -380,7 +380,9 @@ int cie_mixed_attention(void* o, const void* q,
  *                   valid for the batch (cu_seqlens, kv_lens, slot_ids),
  *                   shape and partials_bytes it was made with.  A planned
  *                   call whose B, max_seqlen's query tiles, H_q, H_kv or
- *                   partials budget differ from the plan's writes nothing
+ *                   partials budget differ from the plan's, or whose total_T
+ *                   or max_seqlen makes items of another kind (wide ones from
+ *                   a number of rows on), writes nothing
  *                   and raises CIE_ERRBIT_PLAN.  A batch with more items than
  *                   the plan holds (only sequences that overlap in
  *                   cu_seqlens can have them) gets an empty plan and

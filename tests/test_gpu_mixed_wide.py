@@ -1,11 +1,10 @@
 """Wide launches of the mixed kernel (enough prefill rows to fill the chip) against the oracle.
 
-Each case is sized past the rule that makes a launch wide — tiles of
-16 * floor(8 / G) rows times kv heads, at least 96 at D = 128 and 128 * min(G, 4)
-at D = 64 — and compared with the fp32 oracle, planned and unplanned (which
-must agree bit for bit), at the edges of the tiles: lengths of a whole tile,
-one row more and less, chunks of one and two column tiles a wave, sequences
-that split their keys and decode rows beside them."""
+Every case here asserts from its plan that the launch is wide.  It is compared
+with the fp32 oracle, planned and unplanned (which must agree bit for bit), at
+the edges of the tiles: lengths of a whole tile (16 * floor(8 / G) rows), one row
+more and less, chunks of one and two column tiles a wave, items of half the
+columns, sequences that split their keys and decode rows beside them."""
 import pytest
 import torch
 
@@ -17,13 +16,22 @@ from tests.gpu_helpers import DEV, bits, err_word, note, oracle_mixed
 pytestmark = pytest.mark.gpu
 
 
-def _wide(case, h_q, h_kv, d):
-    rows = 16 * (8 // (h_q // h_kv))
-    tiles = case.T * h_kv // rows
-    return tiles >= (96 if d == 128 else 128 * min(4, h_q // h_kv))
+def _word(plan):
+    """Header word 6 of a mixed plan: 16 * column tiles an item + 16-row blocks a tile, 0 if not wide."""
+    return int(plan[6])
 
 
-def _run(case, h_q, max_seqlen=None, poison=False, rows=slice(None), bad_v=()):
+def _most_chunks(plan):
+    """The most chunks that a query tile of the plan has."""
+    n, (ct, m) = int(plan[0]), divmod(_word(plan), 16)
+    items = plan[8:8 + 8 * n].view(n, 8).cpu()
+    _, count = torch.unique(items[:, 0] * (1 << 20) + items[:, 1], return_counts=True)
+    g = int(plan[4]) // int(plan[5])
+    return int(count.max()) // (2 if m * g > ct else 1)
+
+
+def _run(case, h_q, max_seqlen=None, poison=False, rows=slice(None), bad_v=(), chunks=1,
+         half=False):
     c = case.to(DEV)
     kp, vp = c.k_pool.clone(), c.v_pool.clone()
     if poison:  # pool rows past each sequence's end hold NaN (as uninitialised memory may)
@@ -43,6 +51,8 @@ def _run(case, h_q, max_seqlen=None, poison=False, rows=slice(None), bad_v=()):
         row[:, 0::2], row[:, 1::2] = float("inf"), float("nan")
     ms = max_seqlen or int(case.new_lens.max())
     plan = mixed_plan(kp, c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table, ms, case.T, h_q, err=err)
+    assert _word(plan) // 16 == (4 if half else 8), "not the items that this case is for"
+    assert _most_chunks(plan) >= chunks
     o = [mixed_gqa_attention(c.q, kp, vp, ms, c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table, err=err,
                              plan=p) for p in (plan, None)]
     torch.cuda.synchronize()
@@ -60,7 +70,20 @@ CASES = {
     "d64-g1": (8, 8, 64, 16, [0, 3, 200, 64], [900, 129, 1100, 16]),
     "d64-g2": (8, 4, 64, 32, [0, 31, 1500], [2000, 65, 2200]),
     "d64-g7": (14, 2, 64, 16, [0, 15, 600, 40, 1000], [2100, 15, 1990, 1, 1]),
-    "d64-g5": (20, 4, 64, 16, [10, 0], [17, 2200]),
+    "d64-g5": (20, 4, 64, 16, [10, 0], [17, 2500]),
+    "d64-g3": (24, 8, 64, 16, [10, 0], [33, 2100]),
+    "d64-g4": (16, 4, 64, 16, [0, 100], [3000, 257]),
+    "d64-g6": (24, 4, 64, 16, [0, 100], [2100, 33]),
+    "d64-g8": (32, 4, 64, 16, [0, 100], [1570, 17]),
+    "d128-g3": (24, 8, 128, 16, [0, 100, 9], [300, 33, 70]),
+    "d128-g6": (24, 4, 128, 16, [0, 100, 9], [300, 33, 70]),
+    # items of half the columns: one long prompt makes most of few columns
+    "d128-g7-half": (14, 2, 128, 16, [0, 700, 33, 90], [630, 17, 16, 1]),
+    "d128-g1-half": (8, 8, 128, 16, [0, 500, 0, 7], [1100, 1, 63, 65]),
+    "d128-g2-half": (16, 8, 128, 32, [30, 500], [550, 33]),
+    "d128-g3-half": (12, 4, 128, 16, [30, 500], [750, 17]),
+    "d128-g5-half": (10, 2, 128, 16, [30, 500], [900, 16]),
+    "d128-g8-half": (16, 2, 128, 16, [30, 500], [600, 2]),
 }
 
 
@@ -68,22 +91,46 @@ CASES = {
 def test_wide_launch_matches_the_oracle(native_lib, name):
     h_q, h_kv, d, ps, prior, new = CASES[name]
     case = inputs.make_case(prior, new, h_q=h_q, h_kv=h_kv, d=d, page_size=ps, seed=91)
-    assert _wide(case, h_q, h_kv, d)
     note(f"wide {name}")
-    o, err = _run(case, h_q, poison=True)
+    o, err = _run(case, h_q, poison=True, half=name.endswith("half"))
     assert err == 0
     want, written = oracle_mixed(case)
     assert_attn_close(o[written], want[written], what=name)
 
 
+# h_q, h_kv, d, rows, max_seqlen (None: the rows), column tiles an item (0: 16-row tiles)
+LINES = [
+    (8, 8, 64, 1536, None, 0), (8, 8, 64, 1537, None, 8),
+    (16, 8, 64, 2048, None, 0), (16, 8, 64, 2049, None, 8),
+    (24, 8, 64, 2048, None, 0), (24, 8, 64, 2049, None, 8),
+    (14, 2, 64, 3510, None, 0), (14, 2, 64, 3511, None, 8),
+    (32, 8, 128, 256, None, 0), (32, 8, 128, 257, None, 8),
+    (14, 2, 128, 585, None, 0), (14, 2, 128, 586, None, 4), (14, 2, 128, 586, 256, 8),
+    (14, 2, 128, 877, None, 4), (14, 2, 128, 878, None, 8),
+    (19, 19, 128, 500, None, 4), (20, 4, 128, 410, None, 8),
+]
+
+
+@pytest.mark.parametrize("h_q,h_kv,d,rows,max_seqlen,ct", LINES)
+def test_wide_lines(native_lib, h_q, h_kv, d, rows, max_seqlen, ct):
+    """The launches on either side of each line: columns (rows x q heads) a launch is wide
+    from, and those up to which few heads' items hold half the columns."""
+    pages = -(-rows // 16)
+    pool = torch.zeros(pages, h_kv, 16, d, dtype=torch.float16, device=DEV)
+    i64 = dict(dtype=torch.int64, device=DEV)
+    plan = mixed_plan(pool, torch.tensor([0, rows], **i64), torch.zeros(1, **i64), torch.zeros(1, **i64),
+                      torch.arange(pages, **i64)[None], max_seqlen or rows, rows, h_q)
+    g = h_q // h_kv
+    assert _word(plan) == (ct * 16 + max(1, ct // g) if ct else 0)
+
+
 def test_wide_launch_splits_long_tiles(native_lib):
     """One long chunk over a long prefix beside short ones: its tiles are far above
-    the average share of keys and split in two; with no partials budget the same
+    the average share of keys and split; with no partials budget the same
     tiles run whole, and both match the oracle."""
     case = inputs.make_case([6000, 0, 0], [300, 200, 300], d=128, seed=92)
-    assert _wide(case, 14, 2, 128)
     note("wide split")
-    o, err = _run(case, 14)
+    o, err = _run(case, 14, chunks=2)
     assert err == 0
     want, written = oracle_mixed(case)
     assert_attn_close(o[written], want[written], what="split")
@@ -98,7 +145,6 @@ def test_wide_launch_of_many_sequences(native_lib):
     """More than 64 sequences (the block plan), most of them decode rows."""
     new = [1 if i % 3 else 29 for i in range(100)]
     case = inputs.make_case([(i * 37) % 400 for i in range(100)], new, d=128, seed=93)
-    assert _wide(case, 14, 2, 128)
     note("wide block plan")
     o, err = _run(case, 14)
     assert err == 0
@@ -119,9 +165,11 @@ def test_wide_launch_past_max_seqlen(native_lib):
 
 SPLITS = {
     # few rows over long prefixes: tiles of up to 8 chunks, the partial last tile among them
-    "d128-g7": (14, 2, 128, [9000, 6001, 0, 1500], [770, 30, 17, 1]),
+    "d128-g7": (14, 2, 128, [9000, 6001, 0, 1500], [900, 30, 17, 1]),
+    "d128-g7-half": (14, 2, 128, [9000, 6001, 0, 1500], [670, 30, 17, 1]),
+    "d128-g1-half": (8, 8, 128, [9000, 6001, 0], [1200, 3, 17]),
     "d128-g4": (32, 8, 128, [8015, 700, 3000], [290, 3, 1]),
-    "d64-g1": (8, 8, 64, [7000, 0, 2000], [1501, 70, 1]),
+    "d64-g1": (8, 8, 64, [7000, 0, 2000], [1801, 70, 1]),
 }
 
 
@@ -132,7 +180,7 @@ def test_wide_launch_of_long_prefixes(native_lib, name):
     h_q, h_kv, d, prior, new = SPLITS[name]
     case = inputs.make_case(prior, new, h_q=h_q, h_kv=h_kv, d=d, seed=95)
     note(f"wide long prefixes {name}")
-    o, err = _run(case, h_q)
+    o, err = _run(case, h_q, chunks=3, half=name.endswith("half"))
     assert err == 0
     want, written = oracle_mixed(case)
     assert_attn_close(o[written], want[written], what=name)
@@ -148,12 +196,13 @@ def test_wide_launch_of_long_prefixes(native_lib, name):
 MASKED = {  # h_q, h_kv, d, prior, new
     "d64-g1": (8, 8, 64, [0, 37, 2000], [700, 500, 420]),
     "d64-g2": (16, 8, 64, [0, 37, 2000], [700, 600, 800]),
-    "d64-g3": (24, 8, 64, [0, 37, 2000], [700, 600, 400]),
+    "d64-g3": (24, 8, 64, [0, 37, 2000], [900, 700, 500]),
     "d128-g1": (8, 8, 128, [0, 37, 3000], [900, 700, 500]),
     "d128-g2": (16, 8, 128, [0, 37, 3000], [400, 300, 200]),
     "d128-g4": (32, 8, 128, [0, 37, 3000], [200, 170, 130]),
     "d128-g3": (24, 8, 128, [0, 37, 3000], [200, 170, 130]),
     "d128-g7": (14, 2, 128, [0, 37, 3000], [500, 450, 300]),
+    "d128-g1-half": (8, 8, 128, [0, 37, 3000], [900, 300, 100]),
 }
 
 
@@ -167,9 +216,10 @@ def test_wide_launch_keeps_masked_values_out(native_lib, name):
     # the last block of a wide tile, the second block of one (its first row), the last row
     first = [16 * m - 1 + 16 * m, 16 if m > 1 else 32, new[2] - 1]
     note(f"wide masked {name}")
-    clean, err = _run(case, h_q)
+    half = name.endswith("half")
+    clean, err = _run(case, h_q, half=half)
     assert err == 0
-    bad, err = _run(case, h_q, bad_v=list(enumerate(first)))
+    bad, err = _run(case, h_q, bad_v=list(enumerate(first)), half=half)
     assert err == 0
     for b, j in enumerate(first):
         t0 = int(case.cu_seqlens[b])
