@@ -97,6 +97,7 @@ _SIGNATURES = {
          _c_i64, _c_ptr, _c_ptr],
     ),
     "cie_mixed_partials_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "cie_mixed_default_partials_bytes": (_c_i64, [_c_i64] * 5),
     "cie_mixed_plan_bytes": (_c_i64, [_c_i64, _c_i64]),
     "cie_mixed_plan": (
         ctypes.c_int,

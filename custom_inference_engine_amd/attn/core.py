@@ -463,7 +463,7 @@ def mixed_plan(k_cache, cu_seqlens, kv_lens, slot_ids, block_table, max_seqlen: 
     _require(n > 0, "batch too large for a mixed plan")
     plan = torch.empty(n // 4, dtype=torch.int32, device=dev)
     if partials_bytes is None:
-        partials_bytes = lib.cie_mixed_partials_bytes(int(total_T), num_heads, D)
+        partials_bytes = lib.cie_mixed_default_partials_bytes(int(total_T), int(max_seqlen), num_heads, H_kv, D)
     _native.check(
         lib.cie_mixed_plan(
             plan.data_ptr(), n, cu_seqlens.data_ptr(), kv_lens.data_ptr(), slot_ids.data_ptr(), B,
@@ -484,9 +484,10 @@ def mixed_gqa_attention(q, k, v, max_seqlen: int, cu_seqlens, kv_lens, slot_ids,
     prior lengths; row i of sequence b attends keys [0, kv_lens[b] + i].
     Rows outside every sequence are left as ``torch.empty_like`` leaves them.
     ``partials_bytes`` is the budget of split-chunk partial state (default
-    ``cie_mixed_partials_bytes``: per q head, the larger of 2 rows per token
-    and 16 rows for each of the first 64 tokens, so the decode rows of a
-    small batch can all split); sequences whose split tiles do not fit it
+    ``cie_mixed_default_partials_bytes``: per q head, the larger of 2 rows per
+    token and 16 rows for each of the first 64 tokens, so the decode rows of a
+    small batch can all split, and in launches of enough rows for wide tiles 8
+    rows for each of the first 2,048 tokens, 1,024 at D = 128); sequences whose split tiles do not fit it
     run unsplit, with the same results.
     ``plan``: the step's ``mixed_plan`` (same batch, ``total_T``, heads and
     budget); ``cu_seqlens``, ``kv_lens`` and ``slot_ids`` are then read from it.
@@ -509,7 +510,7 @@ def mixed_gqa_attention(q, k, v, max_seqlen: int, cu_seqlens, kv_lens, slot_ids,
     if B == 0 or total_T == 0 or int(max_seqlen) == 0:
         return o
     if partials_bytes is None:
-        partials_bytes = lib.cie_mixed_partials_bytes(total_T, H_q, D)
+        partials_bytes = lib.cie_mixed_default_partials_bytes(total_T, int(max_seqlen), H_q, H_kv, D)
     _require(partials_bytes >= 0, "partials_bytes must be >= 0")
     partials = torch.empty(partials_bytes, dtype=torch.uint8, device=dev)
     n_ctr = lib.cie_mixed_counters(B, H_kv, int(max_seqlen))

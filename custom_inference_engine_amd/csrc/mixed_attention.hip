@@ -1656,50 +1656,6 @@ static int64_t mixed_partial_rows(int64_t bytes, int64_t D) {
 // prefill: 101.8 us at 2 rows per token, 56.9 at 16).
 constexpr int64_t kDefaultRowsPerToken = 2;
 constexpr int64_t kDefaultChunkedTokens = 64;
-// Wide tiles (from the smallest launches that have them: wide_rule) split up to
-// kWideMaxChunks times where a few hundred rows attend thousands of keys: 8 rows
-// for each of the first 2,048 tokens (D = 128, its rows twice as long: 1,024;
-// 136 MB at 32 heads).  512 tokens over 8,000 keys (14 / 2 heads, D = 128): 163 us
-// unsplit, as 2 rows per token leave it, 91 at 8; 2,048 over 8,000 (8 / 8 heads,
-// D = 64) 117 us with 4 rows, which make three uneven chunks a tile of two.
-constexpr int64_t kDefaultWideRowsPerToken = 8;
-static int64_t default_wide_rows(int64_t total_T, int64_t D) {
-  const int64_t from = D <= 64 ? 1100 : 128, most = D <= 64 ? 2048 : 1024;
-  return total_T < from ? 0 : kDefaultWideRowsPerToken * (total_T < most ? total_T : most);
-}
-
-}  // namespace cie
-
-using namespace cie;
-
-extern "C" int64_t cie_mixed_partials_bytes(int64_t total_T, int64_t H_q, int64_t D) {
-  if (total_T < 0 || H_q <= 0 || D <= 0 || total_T > ((int64_t)1 << 40) / H_q) return -1;
-  const int64_t per_token = kDefaultRowsPerToken * total_T;
-  const int64_t wide = default_wide_rows(total_T, D);
-  const int64_t chunked = kMaxChunks * (total_T < kDefaultChunkedTokens ? total_T : kDefaultChunkedTokens);
-  int64_t rows = (per_token > chunked ? per_token : chunked);
-  rows = (rows > wide ? rows : wide) * H_q;
-  if (rows > kMaxPartRows) rows = kMaxPartRows;
-  // (a multiple of 256, and the alignment of the layout's regions, which
-  // mixed_partial_rows takes off, on top: a batch of exactly these rows fits)
-  return (rows * 4 * (D + 2) + 255) / 256 * 256 + 3 * 256;
-}
-
-extern "C" int64_t cie_mixed_counters(int64_t B, int64_t H_kv, int64_t max_seqlen) {
-  if (B < 0 || H_kv <= 0 || max_seqlen < 0) return -1;
-  // arrival words, then as many stale words (arrive_last)
-  return 2 * B * H_kv * ((max_seqlen + 15) / 16) * kMaxColGroups;
-}
-
-#ifdef CIE_MIXED_TRACE
-// Trace builds only: where the mixed kernel stamps its phases (device buffer
-// of 16 uint64 per (kv head, item); NULL turns the stamps off).
-extern "C" int cie_mixed_trace_buffer(void* buf) {
-  uint64_t* p = static_cast<uint64_t*>(buf);
-  return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_mixed_trace), &p, sizeof(p));
-}
-#endif
-
 // Whether a launch is wide (see wide_tiles.h), from its columns (row, q head) if
 // every row is prefill: a wide item runs a longer serial loop than a narrow one,
 // so a launch is wide where narrow items need one more round of the CUs than the
@@ -1723,21 +1679,83 @@ extern "C" int cie_mixed_trace_buffer(void* buf) {
 // (8 / 8 heads, D = 64, 95 chunks of 17 rows over 2,000 keys 158 / 91; 32 / 8, D =
 // 128, 71 of 5 160 / 156; 400 decode rows of 100 keys 78 / 63).
 constexpr int64_t kWideLongRatio = 20;
-static void wide_rule(MixedParams& p, int64_t max_seqlen, int64_t D) {
-  if (!(D <= 64 ? has_wide<64>() : has_wide<128>())) return;
-  const int64_t columns = p.total_T * p.H_q;
-  const int64_t line = D > 64 ? 8192 : p.G == 1 ? 12288 : p.G == 2 ? 32768 : 49152;
-  if (columns <= line) return;
-  const int64_t longest = max_seqlen < p.total_T ? max_seqlen : p.total_T;
+struct WideShape {
+  int m, ct;  // 16-row blocks of a tile and column tiles of an item; 0, 0: not wide
+};
+static WideShape wide_rule(int64_t total_T, int64_t max_seqlen, int64_t H_q, int64_t G, int64_t D) {
+  if (!(D <= 64 ? has_wide<64>() : has_wide<128>())) return {0, 0};
+  const int64_t columns = total_T * H_q;
+  const int64_t line = D > 64 ? 8192 : G == 1 ? 12288 : G == 2 ? 32768 : 49152;
+  if (columns <= line) return {0, 0};
+  const int64_t longest = max_seqlen < total_T ? max_seqlen : total_T;
   const int ct = D > 64 && columns <= 12288 && columns < kWideLongRatio * longest ? kWideColTiles / 2
                                                                                   : kWideColTiles;
-  const int m = ct > p.G ? ct / p.G : 1;  // (G <= 8)
+  const int m = ct > G ? ct / (int)G : 1;  // (G <= 8)
   // a tile's partial region is addressed in 31 bits
-  if ((int64_t)16 * m * p.H_q * kWideMaxChunks * D * 4 > 0x7fffffff) return;
-  p.wide_m = m;
-  p.wide_ct = ct;
-  p.wide_wg = mixed_workgroups(p.H_kv, D <= 64 ? wide_waves_per_simd<64>() : wide_waves_per_simd<128>());
+  if (16 * m * H_q * kWideMaxChunks * D * 4 > 0x7fffffff) return {0, 0};
+  return {m, ct};
 }
+
+// A wide launch (wide_rule) may hold 8 rows for each of its first 2,048 tokens (D =
+// 128, whose rows are twice as long: 1,024; 136 MB at 32 heads): its tiles split up
+// to kWideMaxChunks times where a few hundred rows attend thousands of keys.  512
+// tokens over 8,000 keys (14 / 2 heads, D = 128): 163 us unsplit, as 2 rows per token
+// leave it, 91 at 8; 2,048 over 8,000 (8 / 8 heads, D = 64) 117 us with 4 rows, which
+// make three uneven chunks a tile of two, 88 with 8.
+constexpr int64_t kDefaultWideRowsPerToken = 8;
+static int64_t default_wide_rows(int64_t total_T, int64_t D) {
+  const int64_t most = D <= 64 ? 2048 : 1024;
+  return kDefaultWideRowsPerToken * (total_T < most ? total_T : most);
+}
+
+// Bytes of a budget of `rows` rows: a multiple of 256, and the alignment of the
+// layout's regions, which mixed_partial_rows takes off, on top (a batch of exactly
+// these rows fits).
+static int64_t budget_bytes(int64_t rows, int64_t D) {
+  if (rows > kMaxPartRows) rows = kMaxPartRows;
+  return (rows * 4 * (D + 2) + 255) / 256 * 256 + 3 * 256;
+}
+static int64_t default_rows(int64_t total_T) {  // (per q head)
+  const int64_t per_token = kDefaultRowsPerToken * total_T;
+  const int64_t chunked = kMaxChunks * (total_T < kDefaultChunkedTokens ? total_T : kDefaultChunkedTokens);
+  return per_token > chunked ? per_token : chunked;
+}
+
+}  // namespace cie
+
+using namespace cie;
+
+extern "C" int64_t cie_mixed_partials_bytes(int64_t total_T, int64_t H_q, int64_t D) {
+  if (total_T < 0 || H_q <= 0 || D <= 0 || total_T > ((int64_t)1 << 40) / H_q) return -1;
+  return budget_bytes(default_rows(total_T) * H_q, D);
+}
+
+extern "C" int64_t cie_mixed_default_partials_bytes(int64_t total_T, int64_t max_seqlen, int64_t H_q,
+                                                    int64_t H_kv, int64_t D) {
+  if (max_seqlen < 0 || H_kv <= 0 || H_q % H_kv != 0) return -1;
+  const int64_t bytes = cie_mixed_partials_bytes(total_T, H_q, D);
+  const int64_t G = H_q / H_kv;
+  // (a launch refuses other head dims and groups)
+  if (bytes < 0 || (D != 64 && D != 128) || G < 1 || G > 8) return bytes;
+  if (wide_rule(total_T, max_seqlen, H_q, G, D).m == 0) return bytes;
+  const int64_t wide = budget_bytes(default_wide_rows(total_T, D) * H_q, D);
+  return wide > bytes ? wide : bytes;
+}
+
+extern "C" int64_t cie_mixed_counters(int64_t B, int64_t H_kv, int64_t max_seqlen) {
+  if (B < 0 || H_kv <= 0 || max_seqlen < 0) return -1;
+  // arrival words, then as many stale words (arrive_last)
+  return 2 * B * H_kv * ((max_seqlen + 15) / 16) * kMaxColGroups;
+}
+
+#ifdef CIE_MIXED_TRACE
+// Trace builds only: where the mixed kernel stamps its phases (device buffer
+// of 16 uint64 per (kv head, item); NULL turns the stamps off).
+extern "C" int cie_mixed_trace_buffer(void* buf) {
+  uint64_t* p = static_cast<uint64_t*>(buf);
+  return (int)hipMemcpyToSymbol(HIP_SYMBOL(g_mixed_trace), &p, sizeof(p));
+}
+#endif
 
 // Checks of the batch shape shared by the entry points, and the parameters
 // they determine (the budget of partial rows from partials_bytes included).
@@ -1775,7 +1793,11 @@ static int mixed_shape(MixedParams& p, int64_t B, int64_t total_T, int64_t max_s
   // The buffer sets the budget of partial rows: sequences whose split tiles
   // do not fit run unsplit (the plan's pbase).
   p.part_cap = mixed_partial_rows(partials_bytes, D);
-  wide_rule(p, max_seqlen, D);
+  const WideShape w = wide_rule(total_T, max_seqlen, H_q, G, D);
+  p.wide_m = w.m;
+  p.wide_ct = w.ct;
+  if (w.m > 0)
+    p.wide_wg = mixed_workgroups(p.H_kv, D <= 64 ? wide_waves_per_simd<64>() : wide_waves_per_simd<128>());
   return CIE_OK;
 }
 

@@ -339,11 +339,12 @@ int cie_kv_append_tokens_qkv_rope(void* q_out, void* k_pool, void* v_pool,
  *                per q head, the larger of 2 rows per token and 16 rows (a
  *                decode row's most chunks) for each of the first 64 tokens
  *                (about 7.8 MB for 1,052 tokens, 14 heads, D = 64; 3.8 MB
- *                at most below 512 tokens), and, where wide tiles may split
- *                long prefixes, 8 rows for each of the first 2,048 tokens
- *                (D = 64, from 1,100 tokens) or 1,024 (D = 128, from 128);
- *                partials may be NULL with partials_bytes = 0 (nothing
- *                splits).
+ *                at most below 512 tokens); partials may be NULL with
+ *                partials_bytes = 0 (nothing splits).  Launches of many rows
+ *                run wide query tiles, which split long prefixes over more
+ *                workgroups: cie_mixed_default_partials_bytes is the same
+ *                number for the others, and at least 8 rows for each of a
+ *                wide launch's first 2,048 tokens (D = 128: 1,024).
  *   counters   : cie_mixed_counters(B, H_kv, max_seqlen) int32, 16-byte
  *                aligned, zero before the call and left zero by it (an
  *                arrival word and a stale word per query tile and column
@@ -352,6 +353,8 @@ int cie_kv_append_tokens_qkv_rope(void* q_out, void* k_pool, void* v_pool,
  *                stream-ordered)
  */
 int64_t cie_mixed_partials_bytes(int64_t total_T, int64_t H_q, int64_t D);
+int64_t cie_mixed_default_partials_bytes(int64_t total_T, int64_t max_seqlen, int64_t H_q,
+                                         int64_t H_kv, int64_t D);
 int64_t cie_mixed_counters(int64_t B, int64_t H_kv, int64_t max_seqlen);
 int cie_mixed_attention(void* o, const void* q,
                         const void* k_pool, const void* v_pool,

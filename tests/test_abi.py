@@ -24,7 +24,7 @@ def test_header_declares_the_hot_path():
                  "cie_paged_decode_append", "cie_paged_decode_max_splits",
                  "cie_paged_decode_partials_bytes", "cie_mixed_attention",
                  "cie_paged_decode_qkv_rope", "cie_kv_append_tokens_qkv_rope",
-                 "cie_mixed_partials_bytes", "cie_mixed_counters", "cie_abi_version",
+                 "cie_mixed_partials_bytes", "cie_mixed_default_partials_bytes", "cie_mixed_counters", "cie_abi_version",
                  "cie_status_string"):
         assert want in names
 
@@ -72,6 +72,17 @@ def test_workspace_sizes(native_lib):
     assert native_lib.cie_mixed_partials_bytes(28, 14, 64) >= 16 * 28 * 14 * row
     assert native_lib.cie_mixed_partials_bytes(100, 14, 64) >= 16 * 64 * 14 * row
     assert native_lib.cie_mixed_partials_bytes(100, 14, 64) < 16 * 64 * 14 * row + 1024
+    # wide launches: 8 rows for each of the first 2,048 tokens (D = 128: 1,024); the same
+    # as above for launches that are not, whatever their token count
+    default = native_lib.cie_mixed_default_partials_bytes
+    for T, h_q, h_kv, d, wide in ((385, 32, 32, 64, True), (384, 32, 32, 64, False), (2048, 14, 2, 64, False),
+                                  (4096, 14, 2, 64, True), (585, 14, 2, 128, False), (586, 14, 2, 128, True),
+                                  (256, 32, 8, 128, False), (4096, 32, 8, 128, True), (0, 14, 2, 64, False)):
+        plain, n = native_lib.cie_mixed_partials_bytes(T, h_q, d), default(T, T, h_q, h_kv, d)
+        rows = 8 * min(T, 2048 if d == 64 else 1024) * h_q
+        assert plain < 2 * T * h_q * (d + 2) * 4 + 1024 or T < 512
+        assert max(plain, rows * (d + 2) * 4) <= n < max(plain, rows * (d + 2) * 4) + 1024 if wide else n == plain
+    assert default(10, 10, 0, 2, 64) == default(10, 10, 14, 3, 64) == default(-1, 10, 14, 2, 64) == -1
     # an arrival word and a stale word per (tile, column group)
     n = native_lib.cie_mixed_counters(32, 2, 256)
     assert n >= 2 * 32 * 2 * 16 and n % 2 == 0

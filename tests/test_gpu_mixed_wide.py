@@ -186,7 +186,7 @@ def test_wide_launch_of_long_prefixes(native_lib, name):
     assert_attn_close(o[written], want[written], what=name)
     c = case.to(DEV)
     kp, vp = (t.to(DEV) for t in case.appended_pools())
-    full = native_lib.cie_mixed_partials_bytes(case.T, h_q, d)
+    full = native_lib.cie_mixed_default_partials_bytes(case.T, max(new), h_q, h_kv, d)
     for nbytes in (full // 3, 0):
         o = mixed_gqa_attention(c.q, kp, vp, max(new), c.cu_seqlens, c.kv_lens, c.slot_ids, c.block_table,
                                 partials_bytes=nbytes)
