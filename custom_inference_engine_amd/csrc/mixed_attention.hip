@@ -172,14 +172,15 @@ struct MixedParams {
   float* part_l;    // [part_cap]
   float* part_acc;  // [part_cap][D]
   int64_t part_cap;  // partial rows the caller's buffer holds (<= kMaxPartRows)
+  // (here: further down, the 16-row kernels spill 5 to 30 more scalars)
+  int32_t wide_m;  // 16-row blocks of a wide query tile (wide_rule); 0: the launch has none
+  int32_t wide_ct;  // column tiles a wide item holds at most (a column group)
+  int32_t wide_wg;  // workgroups of a wide launch
   int32_t* counters;  // 2 x [B][H_kv][n_qtiles][kMaxColGroups]: arrival words, then stale words
   int64_t pool_page_stride, pool_head_stride, bt_stride, n_pages, total_T;
   int32_t bt_width, n_slots, B, H_q, H_kv, G, page_size, n_qtiles;
   uint32_t g_magic, tpp_magic;  // div_magic(G), div_magic(page_size / 16)
   uint32_t pool_bytes;          // bytes of each pool if under 4 GiB, else 0
-  int32_t wide_m;  // 16-row blocks of a wide query tile (wide_rule); 0: the launch has none
-  int32_t wide_ct;  // column tiles a wide item holds at most (a column group)
-  int32_t wide_wg;  // workgroups of a wide launch
   float scale_log2;
   int32_t* err;
   // planned launches: the step's plan (cie_mixed_plan) and its capacity in

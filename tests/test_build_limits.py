@@ -76,6 +76,19 @@ def test_shipped_mixed_build_plans_its_largest_batch_within_lds(tmp_path):
         assert static + plan <= 160 * 1024, (static, plan)
 
 
+def test_launches_of_16_row_tiles_keep_their_scalars(tmp_path):
+    """The 16-row kernels' scalars are spilled to vector lanes, a few cycles an item each: no
+    more of them than these kernels had before some launches became wide."""
+    res = _compile(tmp_path)
+    assert res.returncode == 0, res.stderr[-3000:]
+    spills = re.findall(r"mixed_attention_kernelILi(\d+)ELb1ELb([01])ELb0EE.*?SGPRs Spill: (\d+)", res.stderr,
+                        flags=re.S)
+    most = {("64", "0"): 47, ("64", "1"): 40, ("128", "0"): 33, ("128", "1"): 27}
+    assert {(d, planned) for d, planned, _ in spills} == set(most)
+    for d, planned, n in spills:
+        assert int(n) <= most[d, planned], (d, planned, n)
+
+
 @pytest.mark.parametrize("waves", [1, 4])
 def test_decode_merge_of_many_splits_fits_its_lds(tmp_path, waves):
     """The merge keeps a float for each of 16 heads x 64 splits and 16 bytes a thread in the
