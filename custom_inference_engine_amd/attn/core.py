@@ -128,7 +128,9 @@ def decode_plan(k_cache, lens, slot_ids, block_table, append: bool = True, num_p
     the grid) and every workgroup's page ids are worked out once here; a
     layer's planned launch then reads its descriptor and page ids in one
     memory round trip.  ``num_programs`` (splits per sequence) sizes the grid
-    at ``B * H_kv * num_programs`` workgroups; by default about one per CU.
+    at ``B * H_kv * num_programs`` workgroups; by default about one per CU, two
+    where ``B * H_kv`` is more than the CUs, and one per (sequence, kv head)
+    where it is more than twice as many.
     Returns an int32 tensor; pass it as ``plan=`` to the decode functions of
     the same step (same ``append`` mode, block table and lengths)."""
     N_PAGES, H_kv, PAGE_SIZE, _ = k_cache.shape

@@ -845,8 +845,8 @@ __device__ __forceinline__ void merge_splits(const DecodeParams& p, const PartRo
 // unplanned one needs two (slot id, then page ids and length).
 //
 // Splits are balanced by length: tau, the smallest tile count per split (at
-// least a tile per wave: more splits would be empty) for which sum_b max(1, ceil(tiles_b / tau)) splits (at most kMaxSplits each)
-// fit the grid's n_wg / H_kv workgroups per kv head, gives sequence b
+// least a tile per wave: more splits would be empty; plan_min_tiles) for which
+// sum_b max(1, ceil(tiles_b / tau)) splits (at most kMaxSplits each) fit the grid's n_wg / H_kv workgroups per kv head, gives sequence b
 // ceil(tiles_b / tau) splits, so the longest sequences no longer set the call
 // when lengths differ.  Equal lengths get equal splits (the unplanned deal).
 // Every workgroup of the plan launch redoes the balance (a few hundred
@@ -862,6 +862,7 @@ struct PlanParams {
   const int64_t* block_table;
   int64_t bt_stride, n_pages;
   int32_t B, H_kv, page_size, bt_width, n_slots, n_wg, append;
+  int32_t min_tiles;  // tau is at least this
   int32_t* err;
 };
 
@@ -964,7 +965,7 @@ __device__ __forceinline__ void plan_wave(const PlanParams& p) {
     for (int off = 1; off < kWave; off <<= 1) c += __shfl_xor(c, off, kWave);
     return c <= n_ph;
   };
-  int lo = max(kPlanWaves, (total + n_ph - 1) / n_ph);
+  int lo = max(p.min_tiles, (total + n_ph - 1) / n_ph);
   hi = max(hi, lo);
   if (!fits(lo)) {  // binary search in (lo, hi]; hi always fits (one split each)
     while (lo + 1 < hi) {
@@ -1038,7 +1039,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_plan_kernel(PlanParams p)
   // 2. the smallest tiles-per-split tau whose splits fit n_wg / H_kv per kv head
   const int n_ph = p.n_wg / p.H_kv;
   auto splits_of = [](int nt, int tau) { return plan_splits(nt, tau); };
-  int lo = kPlanWaves;
+  int lo = p.min_tiles;
   hi = max(hi, lo);
   while (lo < hi) {  // uniform: every thread holds the same bounds
     const int mid = (lo + hi) >> 1;
@@ -1360,17 +1361,34 @@ extern "C" int cie_paged_decode_qkv_rope(
 // ---------------------------------------------------------------------------
 // Planned decode: cie_paged_decode_plan once per decode step, then one
 // planned launch per layer.
+// Workgroups a kv head in one round of the CUs.
+static int64_t plan_round(int64_t H_kv) { return (device_cus() + H_kv - 1) / H_kv; }
+
+// Tiles a split holds at least under the default grid.  With a workgroup a CU or
+// more a split competes with the other sequences, and pays its start and its part
+// in a merge, so only long sequences are split there.  us a call, a split a
+// sequence / splits of 4 tiles or more / of 48 (in brackets 64): 14 / 2 heads, D =
+// 64: 204 sequences of 32-1,024 keys 19.9 / 18.6 / 18.5 [19.4], 131 of 400-3,000
+// 35.1 / 26.8 / 26.6 [26.6], 131 of 96-128 9.2 / 11.2 / 8.8 [8.9]; 28 / 4 65 of 32-1,024
+// 14.0 / 15.4 / 17.0 [13.8]; D = 128, 14 / 2, 131 of 32-1,024 20.9 / 25.9 / 26.6 [20.4],
+// 32 / 8 51 of 32-1,024 31.3 / 28.9 / 28.6 [31.1].
+static int plan_min_tiles(int64_t B, int64_t H_kv) {
+  const int64_t round = plan_round(H_kv);
+  return B <= round ? kPlanWaves : 4 * B < 5 * round ? 64 : 48;
+}
+
 extern "C" int64_t cie_paged_decode_plan_workgroups(int64_t B, int64_t H_kv, int64_t n_splits) {
   if (B <= 0 || H_kv <= 0 || n_splits < 0 || n_splits > kMaxSplits) return -1;
   if (n_splits > 0) return B * H_kv * n_splits;
   // the library's default: about one workgroup per CU (one resident round),
-  // at least one and at most kMaxSplits per (sequence, kv head).  More
-  // sequences than that take whole rounds of CUs: the workgroups past B * H_kv
-  // go to the longest sequences, which would otherwise set the call (200
-  // sequences of 32-1,024 keys: 18.5 us a call on 400 workgroups, 16.9 on 512;
-  // 140 of 128-2,048: 25.3 and 20.8).
-  int64_t per_head = (device_cus() + H_kv - 1) / H_kv;
-  if (per_head < B) per_head = (B + per_head - 1) / per_head * per_head;
+  // at least one and at most kMaxSplits per (sequence, kv head).  Up to twice as
+  // many (sequence, kv head) pairs as CUs take two workgroups a CU: those past
+  // B * H_kv go to the longest sequences, which would otherwise set the call
+  // (plan_min_tiles).  More pairs than that have no sequence long enough to set
+  // it (65 sequences of 32-1,024 keys, 8 kv heads, D = 64: 20.2 us a call on 520
+  // workgroups, 24.2 on three a CU; 99 of 400-3,000, D = 128: 120 and 123).
+  int64_t per_head = plan_round(H_kv);
+  if (per_head < B) per_head = B <= 2 * per_head ? 2 * per_head : B;
   if (per_head > B * kMaxSplits) per_head = B * kMaxSplits;
   return H_kv * per_head;
 }
@@ -1416,6 +1434,8 @@ extern "C" int cie_paged_decode_plan(void* plan, const int64_t* lens, const int6
   q.n_slots = (int32_t)(n_slots > 0x7fffffff ? 0x7fffffff : n_slots);
   q.n_wg = (int32_t)n_workgroups;
   q.append = (int32_t)append;
+  q.min_tiles = n_workgroups == cie_paged_decode_plan_workgroups(B, H_kv, 0) ? plan_min_tiles(B, H_kv)
+                                                                            : kPlanWaves;
   q.err = err;
   hipLaunchKernelGGL(decode_plan_kernel, dim3((unsigned)n_workgroups), dim3(kPlanThreads), 0,
                      static_cast<hipStream_t>(stream), q);

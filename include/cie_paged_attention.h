@@ -185,11 +185,13 @@ int cie_paged_decode_append(void* o, const void* q, void* k_pool, void* v_pool,
  * as the layers' calls, and n_workgroups must be the same for all of them.
  * n_workgroups = cie_paged_decode_plan_workgroups(B, H_kv, n_splits):
  * B * H_kv * n_splits, or with n_splits = 0 the library's default (about
- * one workgroup per CU, or the whole number per CU that gives every (sequence,
- * kv head) at least one); it must lie
+ * one workgroup per CU, two where B * H_kv is more than the CUs, and one per
+ * (sequence, kv head) where it is more than twice as many); it must lie
  * in [B * H_kv, B * H_kv * cie_paged_decode_max_splits()] and be a multiple
- * of H_kv.  Equal lengths give every (sequence, kv head) n_workgroups /
- * (B * H_kv) splits; unequal ones give longer sequences more.  partials:
+ * of H_kv.  Equal lengths give every (sequence, kv head) as many splits as
+ * fit, n_workgroups / (B * H_kv) rounded down, but none of fewer than 4
+ * 16-key tiles (48 or 64 under the default of two workgroups per CU); unequal
+ * ones give longer sequences more.  partials:
  * cie_paged_decode_planned_partials_bytes(n_workgroups, H_q, H_kv, D);
  * counters: 2 * B * H_kv words as for cie_paged_decode.  B <= 1024.
  * Replaces decode_gqa_attention (attn/core.py:13-66) and its grid

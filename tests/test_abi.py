@@ -239,6 +239,11 @@ def test_plan_rejects_what_it_cannot_hold(native_lib):
                                         1024, 64, 64, 6, None, None) == -1
     assert lib.cie_paged_decode_plan_workgroups(4, 2, 65) == -1
     assert lib.cie_paged_decode_plan_workgroups(4, 2, 16) == 128
+    # the default grid: one workgroup a CU (256, also where there is no GPU to ask), two up to
+    # twice as many (sequence, kv head) pairs, then one a pair
+    for B, h_kv, n in ((1, 2, 128), (32, 2, 256), (128, 2, 256), (129, 2, 512), (256, 2, 512), (257, 2, 514),
+                       (65, 8, 520), (33, 8, 512), (22, 12, 264), (23, 12, 528), (1000, 1, 1000)):
+        assert lib.cie_paged_decode_plan_workgroups(B, h_kv, 0) == n, (B, h_kv)
     assert lib.cie_paged_decode_plan_bytes(256) == 256 * (8 + 4 * 64) * 4
 
 

@@ -75,6 +75,28 @@ def test_planned_equals_unplanned_on_equal_lengths(native_lib, make, splits):
     assert torch.equal(o1, o2)
 
 
+@pytest.mark.parametrize("B,least", [(131, 64), (170, 48), (250, 48), (260, None)])
+def test_plan_of_more_sequences_than_workgroups_splits_long_ones_only(native_lib, B, least):
+    """With more (sequence, kv head) pairs than CUs a split holds at least 64 tiles, 48 from
+    five pairs for every four CUs on, and past two pairs a CU no sequence is split."""
+    longest = [1200, 780, 760, 1040, 1010, 1500]  # keys with the new one: 76, 49, 48, 66, 64, 94 tiles
+    lens = [longest[i // 20] if i % 20 == 5 and i < 120 else (i * 7) % 200 for i in range(B)]
+    case = inputs.make_case(lens, seed=71)
+    note(f"plan of {B} sequences")
+    c = case.to(DEV)
+    plan = decode_plan(c.k_pool, c.lens_pool, c.slot_ids, c.block_table, append=True)
+    desc = plan[:plan.numel() // 264 * 8].view(-1, 8).cpu()
+    assert (desc[:, 0] >= 0).sum() <= desc.shape[0]
+    for b, n in enumerate(lens):
+        tiles = n // 16 + 1
+        want = 1 if least is None else max(1, -(-tiles // least))
+        assert set(desc[desc[:, 0] == b][:, 3].tolist()) == {want}, (b, n)
+    kp, vp, o = _fused(case)
+    ko, vo = case.appended_pools()
+    assert torch.equal(bits(kp), bits(ko)) and torch.equal(bits(vp), bits(vo)), "append not bit-exact"
+    assert_attn_close(o, oracle_decode(case), what=f"{B} sequences")
+
+
 def test_planned_plain_decode(native_lib):
     """The plan of the plain op (append=False: lens are attended lengths per sequence)."""
     case = inputs.make_case([10, 900, 2047, 0, 4096, 33], seed=65)
