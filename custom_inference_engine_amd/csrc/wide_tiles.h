@@ -2,34 +2,32 @@
 // workgroup.
 //
 // A wide item is up to 8 column tiles of 16 (row, head) columns, two to each of
-// the workgroup's four waves; every wave streams all of the item's keys against
-// its own columns, so nothing is folded across waves, and the keys are read
-// once per workgroup and staged in LDS.  A narrow item (attn_engine.h) gives
-// every wave all columns and a quarter of the keys: short loops that suit few,
-// latency-bound tiles, but at D = 64 each 64 columns (D = 128: each 16) read
-// their whole prefix from L2, and each item pays its start and its fold.
+// the workgroup's four waves (4 and one, in some launches of few columns:
+// wide_rule); every wave streams all of the item's keys against its own columns,
+// so nothing is folded across waves, and the keys are read once per workgroup and
+// staged in LDS.  A narrow item (attn_engine.h) gives every wave all columns and a
+// quarter of the keys: short loops that suit few, latency-bound tiles, but at D =
+// 64 each 64 columns (D = 128: each 16) read their whole prefix from L2, and each
+// item pays its start and its fold.
 //
-// What bounds it: a wave's 32-key step is a serial chain (operands from LDS,
-// S MFMAs, maximum, exponentials, P.V MFMAs, a barrier a stage) of ~1,300
-// cycles at D = 64 however it is scheduled (with the exponentials taken out
-// 1,160, without the staging and its barrier 920), of which its VALU work is
-// ~500 and its MFMAs 256.  So registers and LDS are kept small enough for three
-// workgroups a CU (two at D = 128), whose waves fill each other's gaps: three
-// waves a SIMD take 1,390 cycles a step each, 463 a wave-step, about the VALU
-// time.  Two column tiles a wave and three waves beat four and two (225 us
-// against 251 for 8,192 tokens, 14 / 2 heads, before the third wave: 190).
-// At D = 128 the K/V stream through L2 adds (57 % hits for 8 kv heads of 5,000
-// keys).  Measured, us a launch with narrow items / wide: 4 x 2,048 new tokens
-// (14 / 2 heads, D = 64) 82 / 64; 1 x 8,192 280 / 178; 8 x 1,024 (8 / 8 heads)
-// 95 / 31; 3 ragged chunks of up to 1,024 over up to 4,096 keys and 13 decode
-// rows (32 / 8 heads, D = 128) 267 / 92; 1 x 8,192 (16 / 4 heads, D = 128)
-// 1,600 / 300 (an S.P.V rate of 880 TFLOP/s).
+// What bounds it: a wave's 32-key step is a serial chain (operands from LDS, S
+// MFMAs, maximum, exponentials, P.V MFMAs, a barrier a stage).  So registers and
+// LDS are kept small enough for three workgroups a CU (two at D = 128), whose
+// waves fill each other's gaps; the MFMA pipes are then busy 23 % of a launch (4 x
+// 2,048 new tokens, 14 / 2 heads, D = 64) to 39 % (1 x 8,192, 16 / 4 heads, D = 128),
+// and a third of the LDS cycles at D = 64, half at D = 128, are bank conflicts; K/V
+// reads hit L2 at 83-95 %.  Measured, us a launch with narrow items / wide
+// (kernel times, profiles/mixed_wide_tiles.md): 4 x 2,048 new tokens (14 / 2 heads,
+// D = 64) 86 / 63; 1 x 8,192 305 / 189; 8 x 1,024 (8 / 8 heads) 95 / 30; chunks of
+// 1,024, 700 and 450 over 4,096, 2,000 and 1,000 keys with 13 decode rows (32 / 8
+// heads, D = 128) 649 / 170; 1 x 8,192 (16 / 4 heads, D = 128) 1,596 / 330 (an S.P.V
+// rate of 830 TFLOP/s).
 //
 // Staging: loads that write LDS (no registers), a stage ahead of its use, into
 // the last of three buffers (D = 128: two stages ahead, four), so one barrier a
 // stage suffices.  K rows keep their 16-byte chunks XORed with the row's low 3
-// bits: an operand read (16 rows, one chunk column) covers every bank.  V is
-// read transposed (ds_read_b64_tr_b16: a lane gets 4 keys of its dim, the P.V
+// bits, so that an operand read (16 rows, one chunk column) spreads over the banks.
+// V is read transposed (ds_read_b64_tr_b16: a lane gets 4 keys of its dim, the P.V
 // operand, with no VALU), 4 rows of 32 bytes a 16-lane group: its chunk pairs
 // are XORed with the row's low 2 bits.
 #pragma once
@@ -38,13 +36,14 @@
 
 namespace cie {
 
-// Keys a stage (D = 128: half as many, its registers hold a stage's loads too).
+// Keys a stage (D = 128: half as many, so that four stages leave room in LDS for two
+// workgroups a CU).
 template <int D>
 constexpr int stage_keys() {
   return D <= 64 ? 64 : 32;
 }
 constexpr int kWideWaves = 4;
-constexpr int kWideColTiles = 8;  // column tiles an item holds at most: 2 a wave
+constexpr int kWideColTiles = 8;  // column tiles an item holds at most: two a wave
 
 // Waves a SIMD holds (and workgroups a CU, and registers: 512 / this a lane).
 template <int D>

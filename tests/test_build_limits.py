@@ -39,6 +39,14 @@ def test_mixed_build_past_the_lds_budget_does_not_compile(tmp_path):
     assert "exceed a workgroup's LDS" in res.stderr
 
 
+@pytest.fixture(scope="module")
+def shipped(tmp_path_factory):
+    """The compiler's remarks on the shipped mixed kernels."""
+    res = _compile(tmp_path_factory.mktemp("shipped"))
+    assert res.returncode == 0, res.stderr[-3000:]
+    return res.stderr
+
+
 def _wide_kernels(stderr, d):
     """Names of the D = d kernels that run wide items (the last template argument)."""
     return set(re.findall(rf"mixed_attention_kernelILi{d}ELb[01]ELb[01]ELb1EE", stderr))
@@ -54,21 +62,19 @@ def test_mixed_build_of_other_wave_counts_has_no_wide_launch(tmp_path, waves):
     assert _wide_kernels(res.stderr, 128)  # always four waves
 
 
-def test_shipped_mixed_build_plans_its_largest_batch_within_lds(tmp_path):
-    res = _compile(tmp_path)
-    assert res.returncode == 0, res.stderr[-3000:]
-    assert len(_wide_kernels(res.stderr, 64)) == len(_wide_kernels(res.stderr, 128)) == 4
+def test_shipped_mixed_build_plans_its_largest_batch_within_lds(shipped):
+    assert len(_wide_kernels(shipped, 64)) == len(_wide_kernels(shipped, 128)) == 4
     sizes = [int(m) for m in re.findall(r"mixed_attention_kernel\w*.*?\n.*?LDS Size \[bytes/block\]: (\d+)",
-                                        res.stderr, flags=re.S)]
+                                        shipped, flags=re.S)]
     if not sizes:  # remarks printed in another order: take every LDS size line of the file
-        sizes = [int(m) for m in re.findall(r"LDS Size \[bytes/block\]: (\d+)", res.stderr)]
+        sizes = [int(m) for m in re.findall(r"LDS Size \[bytes/block\]: (\d+)", shipped)]
     assert sizes
     k_max_seqs = 1024  # kMaxSeqs: the ABI's batch limit for cie_mixed_attention
     plan = k_max_seqs * 8 + (4 * k_max_seqs + k_max_seqs + 1) * 4
     # three wide workgroups a CU at D = 64, two at D = 128 (LDS goes in 1,280 bytes; the
     # plan tables of a wide launch lie in its stages)
     wide = re.findall(r"mixed_attention_kernelILi(\d+)ELb[01]ELb[01]ELb1EE.*?LDS Size \[bytes/block\]: (\d+)",
-                      res.stderr, flags=re.S)
+                      shipped, flags=re.S)
     assert len(wide) == 8
     for d, static in wide:
         assert 160 * 1024 // (-(-int(static) // 1280) * 1280) >= (3 if d == "64" else 2), (d, static)
@@ -76,12 +82,10 @@ def test_shipped_mixed_build_plans_its_largest_batch_within_lds(tmp_path):
         assert static + plan <= 160 * 1024, (static, plan)
 
 
-def test_launches_of_16_row_tiles_keep_their_scalars(tmp_path):
+def test_launches_of_16_row_tiles_keep_their_scalars(shipped):
     """The 16-row kernels' scalars are spilled to vector lanes, a few cycles an item each: no
     more of them than these kernels had before some launches became wide."""
-    res = _compile(tmp_path)
-    assert res.returncode == 0, res.stderr[-3000:]
-    spills = re.findall(r"mixed_attention_kernelILi(\d+)ELb1ELb([01])ELb0EE.*?SGPRs Spill: (\d+)", res.stderr,
+    spills = re.findall(r"mixed_attention_kernelILi(\d+)ELb1ELb([01])ELb0EE.*?SGPRs Spill: (\d+)", shipped,
                         flags=re.S)
     most = {("64", "0"): 47, ("64", "1"): 40, ("128", "0"): 33, ("128", "1"): 27}
     assert {(d, planned) for d, planned, _ in spills} == set(most)
