@@ -1529,8 +1529,9 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
 // then writes the header {items, partial budget (rows), B, query tiles,
 // H_q, H_kv, plan_wide_word, wide_q} and, per item in dealing order, its descriptor
 // {b, query tile, index in tile, t0, slot, rows, prior, partial base}.
-template <int D>
+template <int D, bool kWide>
 __global__ __launch_bounds__(mixed_waves<D>() * kWave) void mixed_plan_kernel(MixedParams p) {
+  if constexpr (!kWide) p.wide_m = 0;  // (known to the compiler, as in the kernel above)
   constexpr int W = mixed_waves<D>();
   constexpr int NTH = W * kWave;
   typedef MixedLds<D, false> Lds;
@@ -1616,14 +1617,19 @@ static int launch_mixed(const MixedParams& p, hipStream_t stream) {
                            : launch_mixed_kernel<D, false, kPlanned, false>(p, stream);
 }
 
-template <int D>
-static int launch_mixed_plan(const MixedParams& p, hipStream_t stream) {
+template <int D, bool kWide>
+static int launch_mixed_plan_kernel(const MixedParams& p, hipStream_t stream) {
   static int64_t st = -1;
-  if (st < 0) st = static_lds_of(mixed_plan_kernel<D>);
+  if (st < 0) st = static_lds_of(mixed_plan_kernel<D, kWide>);
   if (st + (int64_t)mixed_plan_lds(p.B) > device_lds_limit()) return CIE_EUNSUPPORTED;
-  hipLaunchKernelGGL((mixed_plan_kernel<D>), dim3(1), dim3(mixed_waves<D>() * kWave),
+  hipLaunchKernelGGL((mixed_plan_kernel<D, kWide>), dim3(1), dim3(mixed_waves<D>() * kWave),
                      mixed_plan_lds(p.B), stream, p);
   return (int)hipGetLastError();
+}
+template <int D>
+static int launch_mixed_plan(const MixedParams& p, hipStream_t stream) {
+  return p.wide_m > 0 ? launch_mixed_plan_kernel<D, true>(p, stream)
+                      : launch_mixed_plan_kernel<D, false>(p, stream);
 }
 
 // partials of `rows` rows: part_m | part_l | part_acc, each region 256-byte

@@ -91,6 +91,9 @@ def test_launches_of_16_row_tiles_keep_their_scalars(shipped):
     assert {(d, planned) for d, planned, _ in spills} == set(most)
     for d, planned, n in spills:
         assert int(n) <= most[d, planned], (d, planned, n)
+    # their plan kernels know at build time that no tile is wide
+    plans = re.findall(r"mixed_plan_kernelILi(\d+)ELb0EE.*?TotalSGPRs: (\d+)", shipped, flags=re.S)
+    assert len(plans) == 2 and all(int(n) <= {"64": 79, "128": 75}[d] for d, n in plans)
 
 
 @pytest.mark.parametrize("waves", [1, 4])
