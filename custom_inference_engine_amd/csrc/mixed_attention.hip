@@ -914,12 +914,12 @@ __device__ __forceinline__ WideWork wide_work(const MixedParams& p, const SeqInf
 // others' work is done; its keys go to several workgroups, at the price of
 // partials and a merge.  Few tiles for the chip (long prefixes under few rows)
 // split to 1.5 times the share, as many tiles as workgroups or more to 3 times
-// it, where the other tiles fill the gaps.  Measured, us a call with at most two
-// chunks of 3 times the share / so: D = 128: 1,536 tokens over 8,000 (14 / 2
-// heads) 257 / 175, 3 x 512 over 4,000 130 / 100, 768 over 8,000 134 / 100;
-// D = 64, 8 / 8 heads: 2,048 over 8,000 108 / 88; 4 x 2,048 on nothing (14 / 2)
-// 72 / 68.  Chunks of fewer than 16 steps (D = 128: 24) cost more in the merge
-// than they save (1,024 over 2,000: 75 us at 16 steps, 61 at 32).
+// it, where the other tiles fill the gaps.  Measured, us a call with its append
+// (profiles/mixed_wide_tiles.md), at most two chunks of 3 times the share / so: D =
+// 128: 1,536 tokens over 8,000 (14 / 2 heads) 246 / 172, 3 x 512 over 4,000 128 / 104,
+// 512 over 8,000 (32 / 8) 127 / 112; D = 64: 2,048 over 8,000 (8 / 8) 105 / 87; 4 x
+// 2,048 on nothing (14 / 2) 73 / 71.  Chunks of less than the minimum cost more in
+// the merge than they save (D = 128, 32 / 8, 290 over 2,000: 48 at half of it, 43).
 constexpr float kWideShareMin = 1.5f, kWideShareMax = 3.f, kWideShareSlope = 6.f;
 template <int D>
 constexpr int kWideMinSplit = D <= 64 ? 32 : 48;
@@ -1419,9 +1419,9 @@ __attribute__((amdgpu_waves_per_eu(mixed_waves_per_simd<D, kWide>()))) void mixe
   // Item of round q for this workgroup (see the item loop).  A wide launch has
   // several workgroups a CU, workgroups w and w + CUs on the same one; at D = 64
   // the rounds' direction alternates over CUs, so that a CU's workgroups do not
-  // all hold a sequence's longest tiles (4 x 2,048 tokens: 87 us a launch over
-  // workgroups, 75; D = 128, bound by the K/V stream, is slower that way: 312
-  // against 360 for 8,192 tokens of 16 / 4 heads).
+  // all hold a sequence's longest tiles (4 x 2,048 tokens, 14 / 2 heads: 87 us a
+  // call over workgroups, 75 over CUs; D = 128 is slower that way: 8,192 tokens,
+  // 16 / 4 heads, 326 and 358).
   constexpr int kPerCu = kWide && D <= 64 ? wide_waves_per_simd<D>() : 1;
   const int n_cu_r = n_slots_r / kPerCu;
   const int cu_r = kPerCu > 1 ? slot_r % n_cu_r : slot_r;
@@ -1705,10 +1705,10 @@ static WideShape wide_rule(int64_t total_T, int64_t max_seqlen, int64_t H_q, int
 
 // A wide launch (wide_rule) may hold 8 rows for each of its first 2,048 tokens (D =
 // 128, whose rows are twice as long: 1,024; 136 MB at 32 heads): its tiles split up
-// to kWideMaxChunks times where a few hundred rows attend thousands of keys.  512
-// tokens over 8,000 keys (14 / 2 heads, D = 128): 163 us unsplit, as 2 rows per token
-// leave it, 91 at 8; 2,048 over 8,000 (8 / 8 heads, D = 64) 117 us with 4 rows, which
-// make three uneven chunks a tile of two, 88 with 8.
+// to kWideMaxChunks times where a few hundred rows attend thousands of keys.  us a
+// call with 2 rows per token, as other launches have, 4 and 8: 512 tokens over 8,000
+// keys (32 / 8 heads, D = 128) 221, 143, 112; 2,048 over 8,000 (8 / 8, D = 64) 178, 113,
+// 87; 16 rows are no faster.
 constexpr int64_t kDefaultWideRowsPerToken = 8;
 static int64_t default_wide_rows(int64_t total_T, int64_t D) {
   const int64_t most = D <= 64 ? 2048 : 1024;
